@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -696,6 +697,18 @@ struct DevIndex {
   int* col_list = nullptr;
   int* col_nbr = nullptr;  // the neighbour-table rows of col_list's entries, in its order
   std::vector<int> col_off, col_n, lcol_off, lcol_n;  // [2 * level + colour]
+  // the coarsest level with leaves or residual faces: the cycle and the
+  // residual read no restricted value above it
+  int lneed = 0;
+  // the halo cells that relax, the initial guesses and the residual's faces
+  // read, as 2^dim * record + child, by dependency stage (a cell interpolated
+  // from halo cells of stage k - 1 has stage k) and then by level
+  int* halo = nullptr;
+  int* halo_end_d = nullptr;
+  int nstage = 0;
+  std::vector<int> halo_end;  // [stage * (depth + 1) + level]: end of the stage's cells up to that level
+  int* crec = nullptr;        // per level: the first child record (of the next level) of every nonleaf record
+  std::vector<int> crec_off;
   BoxRule* box = nullptr;
   FaceOp* fops = nullptr;
   FaceAvg *hf = nullptr, *fr = nullptr;
@@ -729,6 +742,9 @@ unsigned nb_(long n) { return (unsigned)((n + kB - 1) / kB); }
 constexpr int kUserScalars = 4;
 // largest operation the batched small-operation kernel takes by default
 constexpr long kSmallOp = 1024;
+// restriction in one launch starts at the first level with this many records,
+// in about so many workgroups
+constexpr int kRestrictBase = 64, kRestrictBlocks = 1024;
 
 struct bmg_tree {
   int dim = 2;
@@ -767,6 +783,9 @@ struct bmg_tree {
   void *da = nullptr, *res = nullptr, *tmp = nullptr, *alT[3] = {nullptr, nullptr, nullptr}, *lamT = nullptr;
   double* bcv[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
   bool coef_ready = false;
+  // the level whose boundary pass of da the last cycle left out (-1: none);
+  // only bmg_tree_relax reads what it would have written
+  int da_level = -1;
   TStat* stat = nullptr;
   double *part = nullptr, *scalar = nullptr;
   hipStream_t own_stream = nullptr, stream = nullptr;
@@ -856,7 +875,7 @@ void free_device(bmg_tree* t) {
   drop_graphs(t);
   DevIndex& x = t->ix;
   for (void* p : {(void*)x.nbr, (void*)x.rec_self, (void*)x.rec_child0, (void*)x.rec_ring, (void*)x.colour,
-                  (void*)x.leaf_gs, (void*)x.lvl_leaves, (void*)x.col_list, (void*)x.col_nbr, (void*)x.box, (void*)x.fops, (void*)x.hf, (void*)x.fr,
+                  (void*)x.leaf_gs, (void*)x.lvl_leaves, (void*)x.col_list, (void*)x.col_nbr, (void*)x.halo, (void*)x.halo_end_d, (void*)x.crec, (void*)x.box, (void*)x.fops, (void*)x.hf, (void*)x.fr,
                   (void*)x.fp, (void*)x.fc, (void*)x.fv_gs, (void*)x.fv_d, (void*)x.fc_tmp, (void*)x.lvinfo})
     dfree_(p);
   x = DevIndex();
@@ -894,6 +913,7 @@ void free_device(bmg_tree* t) {
   t->a = t->b = t->res64 = t->lam64 = nullptr;
   t->da = t->res = t->tmp = t->lamT = nullptr;
   t->stat = nullptr; t->part = t->scalar = nullptr;
+  t->da_level = -1;
   t->compiled = false;
   t->coef_ready = false;
   // the frees above are best effort; do not leave their status behind for
@@ -1173,6 +1193,7 @@ int compile(bmg_tree* t) {
     for (auto& g : T.bnd[l]) {
       BoxRule r;
       memset(&r, 0, sizeof r);
+      r.level = l;
       r.ghost = chk(S(l, g.i, g.j, g.k));
       r.src = -1;
       const int gc[3] = {g.i, g.j, g.k};
@@ -1279,6 +1300,134 @@ int compile(bmg_tree* t) {
     }
   });
   clk.mark("compile: tables: face ops");
+  // ghost entries of the rings become box rules (~r), see GhostRule
+  std::vector<int> gbase(D + 1), hbase(D + 1);
+  std::vector<std::vector<int>> rule(D + 1);
+  for (int l = 0; l <= D; l++) {
+    hbase[l] = x.off[l] + x.nA[l];
+    gbase[l] = hbase[l] + (l ? nch * x.n_prolong[l - 1] : 0);
+    rule[l].assign((size_t)((l < D ? x.off[l + 1] : (int)NS) - gbase[l]), -1);
+    for (int r = x.box_off[l]; r < x.box_off[l] + x.box_n[l]; r++)
+      if (box[r].ghost >= gbase[l] && box[r].ghost - gbase[l] < (int)rule[l].size())
+        rule[l][box[r].ghost - gbase[l]] = r;
+  }
+  auto entry = [&](int l, int v) {
+    if (v < gbase[l] || v - gbase[l] >= (int)rule[l].size()) return v;
+    const int r = rule[l][v - gbase[l]];
+    return r >= 0 ? ~r : v;
+  };
+  for (int l = 0; l <= D; l++) {
+    const size_t w0 = (size_t)x.rec_off[l] * NR;
+    par_for((size_t)(x.n_nonleaf[l] + x.n_prolong[l]) * NR, [&](size_t k0, size_t k1) {
+      for (size_t k = k0; k < k1; k++) rring[w0 + k] = entry(l, rring[w0 + k]);
+    });
+  }
+  // the halo cells that anything reads, and their dependency stages
+  x.lneed = D;
+  for (int l = D; l >= 0; l--)
+    if (x.leaf_n[l] || x.face_n[l] || x.n_prolong[l]) x.lneed = l;
+  table<int> halo;
+  {
+    std::vector<size_t> hoff(D + 2, 0);
+    for (int l = 0; l <= D; l++) hoff[l + 1] = hoff[l] + (size_t)(gbase[l] - hbase[l]);
+    if (nrec * (size_t)nch > (size_t)INT_MAX) return bmg::fail(BMG_ERR_UNSUPPORTED, "tree: too many parent records");
+    // 0: not read; then 1 (read), later the stage
+    std::vector<uint8_t> stage(hoff[D + 1], 0);
+    // the halo cell an entry of level l reads: its index, or -1
+    auto halo_of = [&](int l, int v) -> long {
+      if (v < 0) v = box[~v].nterm ? box[~v].src : -1;
+      return v >= hbase[l] && v < gbase[l] ? (long)(hoff[l] + (size_t)(v - hbase[l])) : -1;
+    };
+    auto mark = [&](int l, int v) {
+      const long h = halo_of(l, v);
+      if (h >= 0) __atomic_store_n(&stage[(size_t)h], (uint8_t)1, __ATOMIC_RELAXED);
+    };
+    for (int l = 0; l <= D; l++) {
+      const size_t a0 = (size_t)x.abase[l] * 2 * dim, w0 = (size_t)x.rec_off[l] * NR;
+      par_for((size_t)x.nA[l] * 2 * dim, [&](size_t k0, size_t k1) {
+        for (size_t k = k0; k < k1; k++) mark(l, entry(l, nbr[a0 + k]));
+      });
+      par_for((size_t)x.n_nonleaf[l] * NR, [&](size_t k0, size_t k1) {
+        for (size_t k = k0; k < k1; k++) mark(l, rring[w0 + k]);
+      });
+      par_for((size_t)x.face_n[l], [&](size_t k0, size_t k1) {
+        for (size_t k = k0; k < k1; k++) {
+          const FaceOp& f = fops[(size_t)x.face_off[l] + k];
+          mark(l, entry(l, f.gs));
+          mark(l, entry(l, f.gm));
+        }
+      });
+    }
+    // ring position of term k of child m's interpolation
+    int pos[8][8];
+    for (int m = 0; m < nch; m++)
+      for (int k = 0; k < nch; k++) {
+        int p = 0;
+        for (int d = 0; d < dim; d++) {
+          const int side = (m >> (dim - 1 - d)) & 1, use = (k >> (dim - 1 - d)) & 1;
+          p = p * 3 + 1 + use * (2 * side - 1);
+        }
+        pos[m][k] = p;
+      }
+    auto terms = [&](int l, size_t h, auto&& f) {  // the ring entries halo cell h of level l is interpolated from
+      const size_t r = (size_t)x.rec_off[l - 1] + x.n_nonleaf[l - 1] + h / nch;
+      for (int k = 0; k < nch; k++) f(rring[r * NR + pos[h % nch][k]]);
+    };
+    for (int l = D; l >= 1; l--)
+      par_for(hoff[l + 1] - hoff[l], [&](size_t h0, size_t h1) {
+        for (size_t h = h0; h < h1; h++)
+          if (__atomic_load_n(&stage[hoff[l] + h], __ATOMIC_RELAXED)) terms(l, h, [&](int v) { mark(l - 1, v); });
+      });
+    std::vector<std::vector<int>> items(kSeg);
+    std::vector<std::vector<int>> count(D + 1, std::vector<int>(kSeg, 0));
+    for (int l = 1; l <= D; l++) {
+      par_for(hoff[l + 1] - hoff[l], [&](size_t h0, size_t h1) {
+        for (size_t h = h0; h < h1; h++) {
+          if (!stage[hoff[l] + h]) continue;
+          int s = 0;
+          terms(l, h, [&](int v) {
+            const long q = halo_of(l - 1, v);
+            if (q >= 0) s = std::max(s, (int)stage[(size_t)q]);
+          });
+          stage[hoff[l] + h] = (uint8_t)(s + 1);
+        }
+      });
+      const int r0 = (x.rec_off[l - 1] + x.n_nonleaf[l - 1]) * nch;
+      for (size_t h = 0; h < hoff[l + 1] - hoff[l]; h++)
+        if (const int s = stage[hoff[l] + h]) {
+          items[s - 1].push_back(r0 + (int)h);
+          count[l][s - 1]++;
+        }
+    }
+    x.nstage = 0;
+    while (x.nstage < kSeg && !items[x.nstage].empty()) x.nstage++;
+    x.halo_end.assign((size_t)std::max(1, x.nstage) * (D + 1), 0);
+    int end = 0;
+    for (int k = 0; k < x.nstage; k++) {
+      for (int l = 0; l <= D; l++) x.halo_end[(size_t)k * (D + 1) + l] = end += count[l][k];
+      halo.insert(halo.end(), items[k].begin(), items[k].end());
+    }
+    TRY(upload(&x.halo, halo));
+    TRY(upload(&x.halo_end_d, x.halo_end));
+  }
+  // the children of nonleaf record k of a level are active cells nch k ..
+  // of the next one, so its child records are a run
+  x.crec_off.assign(D + 1, 0);
+  {
+    std::vector<int> crec;
+    for (int l = 0; l < D; l++) {
+      x.crec_off[l] = (int)crec.size();
+      size_t q = 0;
+      for (int k = 0; k <= x.n_nonleaf[l]; k++) {
+        if (k < x.n_nonleaf[l] && rchild[(size_t)x.rec_off[l] + k] != x.off[l + 1] + k * nch) ok = false;
+        while (q < nonleaf[l + 1].size() && nonleaf[l + 1][q] < k * nch) q++;
+        crec.push_back((int)q);
+      }
+    }
+    if (!ok) return bmg::fail(BMG_ERR_ARG, "tree: children out of cache order");
+    TRY(upload(&x.crec, crec));
+  }
+  clk.mark("compile: tables: halo cells");
   // fine-face averages: halo_face (all levels in one launch) and the face
   // restriction of alpha (per level)
   auto fine_avg = [&](int l, const int c[3], int d, int hi, int target) {
@@ -1517,7 +1666,7 @@ int compile(bmg_tree* t) {
           return;
         }
         const size_t ai = (size_t)x.abase[m] + (gs - x.off[m]);
-        for (int k = 0; k < 2 * dim; k++) cnb[e * 2 * dim + k] = nbr[ai * 2 * dim + k];
+        for (int k = 0; k < 2 * dim; k++) cnb[e * 2 * dim + k] = entry(m, nbr[ai * 2 * dim + k]);
       }
     });
     if (bad) return bmg::fail(BMG_ERR_ARG, "tree: colour list entry outside the active cells");
@@ -1535,7 +1684,9 @@ int compile(bmg_tree* t) {
     std::vector<TLevelInfo> li(D + 1);
     for (int l = 0; l <= D; l++)
       li[l] = {x.off[l], x.nA[l], x.abase[l], x.rec_off[l], x.n_nonleaf[l], x.n_prolong[l],
-               x.box_off[l], x.box_n[l], x.leaf_off[l], x.leaf_n[l]};
+               x.box_off[l], x.box_n[l], x.leaf_off[l], x.leaf_n[l],
+               {x.col_off[2 * l], x.col_off[2 * l + 1]}, {x.col_n[2 * l], x.col_n[2 * l + 1]},
+               {x.lcol_off[2 * l], x.lcol_off[2 * l + 1]}, {x.lcol_n[2 * l], x.lcol_n[2 * l + 1]}};
     TRY(upload(&x.lvinfo, li));
   }
   TRY(dalloc_((void**)&x.fc_tmp, sizeof(double) * std::max(1, x.maxfc)));
@@ -1699,7 +1850,7 @@ template <typename T>
 void box(bmg_tree* t, T* f, int bk, int l) {
   const DevIndex& x = t->ix;
   int n = x.box_n[l];
-  if (n) k_t_box<T><<<nb_(n), kB, 0, t->stream>>>(x.box + x.box_off[l], n, f, bct(t), bk, delta(t, l));
+  if (n) k_t_box<T><<<nb_(n), kB, 0, t->stream>>>(x.box + x.box_off[l], n, f, bct(t), bk, t->L0);
 }
 
 template <typename T, int DIM>
@@ -1718,7 +1869,8 @@ void prolong_records(bmg_tree* t, T* f, int l, bool halo) {
   int n = halo ? x.n_prolong[l] : x.n_nonleaf[l];
   const int NR = DIM == 3 ? 27 : 9;
   if (n)
-    k_t_prolong<T, DIM><<<nb_(n), kB, 0, t->stream>>>(x.rec_ring + (size_t)r0 * NR, x.rec_child0 + r0, n, f);
+    k_t_prolong<T, DIM>
+        <<<nb_(n), kB, 0, t->stream>>>(x.rec_ring + (size_t)r0 * NR, x.rec_child0 + r0, n, f, x.box);
 }
 
 template <typename T>
@@ -1732,28 +1884,35 @@ RelaxCoef<T> relax_coef(bmg_tree* t) {
 }
 
 template <typename T, int DIM>
+void pending_boundary(bmg_tree* t);
+
+// one relax of level l (bmg_tree_relax): Jacobi reads the ghosts' stored
+// values, red-black evaluates their rules
+template <typename T, int DIM>
 int relax(bmg_tree* t, int l) {
   const DevIndex& x = t->ix;
   Segs S = level_or_leaf(t, l);
   unsigned nbk = (unsigned)S.first_block[S.n];
   if (!nbk) return BMG_OK;
+  pending_boundary<T, DIM>(t);
   RelaxCoef<T> k = relax_coef<T>(t);
   T* da = F<T>(t->da);
   T* res = F<T>(t->res);
   if (t->smoother == BMG_RELAX_JACOBI) {
     {
       TProf tp(t, seg_cells(S));
-      k_t_relax<T, DIM><<<nbk, kB, 0, t->stream>>>(S, da, F<T>(t->tmp), res, x.nbr, x.colour, k, -1);
+      k_t_relax<T, DIM><<<nbk, kB, 0, t->stream>>>(S, da, F<T>(t->tmp), res, x.nbr, x.box, bct(t), t->L0, k);
     }
     k_t_jacobi<T><<<nbk, kB, 0, t->stream>>>(S, da, F<T>(t->tmp));
   } else if (t->smoother == BMG_RELAX_RBGS) {
     for (int c = 0; c < 2; c++) {
+      // (the stored ghosts, which a Jacobi relax may read next)
       if (c) for (int m = 0; m <= l; m++) box<T>(t, da, BK_HOM, m);
       Segs SC = level_or_leaf_colour(t, l, c);
       unsigned nbc = (unsigned)SC.first_block[SC.n];
       if (nbc) {
         TProf tp(t, seg_cells(SC));
-        k_t_relax<T, DIM><<<nbc, kB, 0, t->stream>>>(SC, da, nullptr, res, x.nbr, x.colour, k, 2);
+        k_t_relax<T, DIM><<<nbc, kB, 0, t->stream>>>(SC, da, nullptr, res, x.nbr, x.box, bct(t), t->L0, k);
       }
     }
   } else
@@ -1778,9 +1937,12 @@ struct Batcher {
     A.rec_self = x.rec_self;
     A.rec_child0 = x.rec_child0;
     A.rec_ring = x.rec_ring;
-    A.nbr = x.nbr;
     A.lvl_leaves = x.lvl_leaves;
-    A.colour = x.colour;
+    A.col_list = x.col_list;
+    A.col_nbr = x.col_nbr;
+    A.halo = x.halo;
+    A.halo_end = x.halo_end_d;
+    A.depth = x.depth;
     A.box = x.box;
     A.fld[0] = f0;
     A.fld[1] = f1;
@@ -1795,16 +1957,17 @@ struct Batcher {
     if (P.n) k_t_ops<T, DIM><<<1, t->ops_block, 0, t->stream>>>(P, A);
     P.n = 0;
   }
-  void push(int code, int level, int arg, int field) {
+  void push(int code, int level, int arg, int field, int stage = 0) {
     if (P.n == kMaxOps) flush();
-    P.op[P.n++] = TOp{(unsigned char)code, (unsigned char)field, (signed char)arg, (unsigned char)level};
+    P.op[P.n++] = TOp{(unsigned char)code, (unsigned char)field, (signed char)arg, (unsigned char)level,
+                      (unsigned char)stage};
   }
   void box(int f, int bk, int l) {
     int n = x.box_n[l];
     if (!n) return;
     if (small(n)) return push(TOP_BOX, l, bk, f);
     flush();
-    k_t_box<T><<<nb_(n), kB, 0, t->stream>>>(x.box + x.box_off[l], n, A.fld[f], A.bc, bk, delta(t, l));
+    k_t_box<T><<<nb_(n), kB, 0, t->stream>>>(x.box + x.box_off[l], n, A.fld[f], A.bc, bk, t->L0);
   }
   void restrict_level(int f, int l) {
     int n = x.n_nonleaf[l];
@@ -1821,7 +1984,64 @@ struct Batcher {
     if (small(n)) return push(TOP_PROLONG, l, halo ? 1 : 0, f);
     flush();
     const int NR = DIM == 3 ? 27 : 9;
-    k_t_prolong<T, DIM><<<nb_(n), kB, 0, t->stream>>>(x.rec_ring + (size_t)r0 * NR, x.rec_child0 + r0, n, A.fld[f]);
+    k_t_prolong<T, DIM>
+        <<<nb_(n), kB, 0, t->stream>>>(x.rec_ring + (size_t)r0 * NR, x.rec_child0 + r0, n, A.fld[f], x.box);
+  }
+  // restriction of f to the levels m1 .. m0 (m1 >= m0): the levels from the
+  // first with kRestrictBase records on in one launch, a workgroup per run of
+  // records (one launch per level cost 2.3 us each on a chain of 6)
+  void restrict_range(int f, int m1, int m0) {
+    int base = m0;
+    while (base < m1 && x.n_nonleaf[base] < kRestrictBase) base++;
+    if (m1 - base >= 1 && !small(x.n_nonleaf[m1])) {
+      flush();
+      RestrictLevels L;
+      memset(&L, 0, sizeof L);
+      L.m0 = base;
+      L.m1 = m1;
+      for (int m = base; m <= m1; m++) {
+        L.rec_off[m] = x.rec_off[m];
+        L.n[m] = x.n_nonleaf[m];
+        L.crec_off[m] = x.crec_off[m];
+      }
+      const int n = x.n_nonleaf[base];
+      L.per_block = std::max(1, n / kRestrictBlocks);
+      k_t_restrict_tree<T, DIM><<<(unsigned)((n + L.per_block - 1) / L.per_block), kB, 0, t->stream>>>(
+          L, x.rec_self, x.rec_child0, x.crec, A.fld[f]);
+      m1 = base - 1;
+    }
+    for (int m = m1; m >= m0; m--) restrict_level(f, m);
+  }
+  // what the cycle and the residual read of tree_boundary_level ({f}, l):
+  // the restricted values down to the coarsest level with leaves and the
+  // halo cells, a launch per dependency stage; ghosts are evaluated by
+  // their readers
+  void boundary(int f, int bk, int l) {
+    if (t->topo.full()) return;
+    if (l - 1 >= x.lneed) restrict_range(f, l - 1, x.lneed);
+    for (int k = 0; k < x.nstage; k++) {
+      const int i0 = k ? x.halo_end[(size_t)(k - 1) * (x.depth + 1) + x.depth] : 0;
+      const int n = x.halo_end[(size_t)k * (x.depth + 1) + l] - i0;
+      if (n <= 0) continue;
+      if (small(n)) {
+        push(TOP_HALO, l, bk, f, k);
+        continue;
+      }
+      flush();
+      k_t_children<T, DIM><<<nb_(n), kB, 0, t->stream>>>(x.halo + i0, n, x.rec_ring, x.rec_child0, A.fld[f], x.box,
+                                                         A.bc, bk, t->L0);
+    }
+  }
+  // bilinear into the children of the nonleaf cells of level l
+  void children(int f, int bk, int l) {
+    const int n = x.n_nonleaf[l], NR = DIM == 3 ? 27 : 9;
+    if (!n) return;
+    if (small(n)) return push(TOP_CHILDREN, l, bk, f);
+    flush();
+    k_t_children<T, DIM><<<nb_((long)n << DIM), kB, 0, t->stream>>>(nullptr, n << DIM,
+                                                                   x.rec_ring + (size_t)x.rec_off[l] * NR,
+                                                                   x.rec_child0 + x.rec_off[l], A.fld[f], x.box, A.bc,
+                                                                   bk, t->L0);
   }
   // tree_boundary_level ({f}, l) (l < 0: depth)
   void tree_boundary(int f, int bk, int l) {
@@ -1859,49 +2079,25 @@ struct Batcher {
         push(TOP_JACOBI, l, 0, 0);
       } else {
         push(TOP_RELAX, l, 0, 0);
-        for (int m = 0; m <= l; m++) box(0, BK_HOM, m);
         push(TOP_RELAX, l, 1, 0);
       }
       return BMG_OK;
     }
     flush();
-    Segs S = level_or_leaf(t, l);
-    unsigned nbk = (unsigned)S.first_block[S.n];
-    if (!nbk) return BMG_OK;
     T* da = A.fld[0];
+    for (int c = 0; c < 2; c++) {
+      Segs SC = level_or_leaf_colour(t, l, c);
+      unsigned nbc = (unsigned)SC.first_block[SC.n];
+      if (!nbc) continue;
+      TProf tp(t, seg_cells(SC));
+      k_t_relax<T, DIM><<<nbc, kB, 0, t->stream>>>(SC, da, jac ? A.fld[2] : nullptr, A.res, x.nbr, x.box, A.bc, t->L0,
+                                                   A.k);
+    }
     if (jac) {
-      {
-        TProf tp(t, seg_cells(S));
-        k_t_relax<T, DIM><<<nbk, kB, 0, t->stream>>>(S, da, A.fld[2], A.res, x.nbr, x.colour, A.k, -1);
-      }
-      k_t_jacobi<T><<<nbk, kB, 0, t->stream>>>(S, da, A.fld[2]);
-    } else {
-      for (int c = 0; c < 2; c++) {
-        if (c) {
-          for (int m = 0; m <= l; m++) box(0, BK_HOM, m);
-          flush();
-        }
-        Segs SC = level_or_leaf_colour(t, l, c);
-        unsigned nbc = (unsigned)SC.first_block[SC.n];
-        if (nbc) {
-          TProf tp(t, seg_cells(SC));
-          k_t_relax<T, DIM><<<nbc, kB, 0, t->stream>>>(SC, da, nullptr, A.res, x.nbr, x.colour, A.k, 2);
-        }
-      }
+      Segs S = level_or_leaf(t, l);
+      k_t_jacobi<T><<<(unsigned)S.first_block[S.n], kB, 0, t->stream>>>(S, da, A.fld[2]);
     }
     return BMG_OK;
-  }
-  // restriction (res) of mg_cycle (tree_restriction), on field f
-  void restriction_res(int f) {
-    int D = x.depth;
-    if (t->topo.full()) {
-      box(f, BK_SYM, D);
-      for (int l = D - 1; l >= 0; l--) {
-        restrict_level(f, l);
-        box(f, BK_SYM, l);
-      }
-    } else
-      tree_boundary(f, BK_SYM, -1);
   }
 };
 
@@ -1911,8 +2107,11 @@ void residual_kernels(bmg_tree* t) {
   const DevIndex& x = t->ix;
   {
     Batcher<double, DIM> B(t, t->a, nullptr, nullptr);
-    B.tree_boundary(0, BK_A, -1);
+    B.boundary(0, BK_A, x.depth);
     B.flush();
+    // the ghosts that the face fluxes read, every level with faces
+    const int r0 = x.box_off[x.lneed], n = x.box_off[x.depth] + x.box_n[x.depth] - r0;
+    if (n) k_t_box<double><<<nb_(n), kB, 0, t->stream>>>(x.box + r0, n, t->a, bct(t), BK_A, t->L0);
   }
   const double* al[3] = {nullptr, nullptr, nullptr};
   if (t->alpha_field)
@@ -2036,17 +2235,21 @@ int cycle_kernels(bmg_tree* t, int nrelax, int minlevel, int maxlevel) {
   const DevIndex& x = t->ix;
   T* da = F<T>(t->da);
   Batcher<T, DIM> B(t, da, F<T>(t->res), F<T>(t->tmp));
-  B.restriction_res(1);
   minlevel = std::min(minlevel, maxlevel);
+  // restriction (res) of mg_cycle: relax reads res in the cells it relaxes,
+  // so neither levels above minlevel nor halo cells nor ghosts
+  if (x.depth > minlevel) B.restrict_range(1, x.depth - 1, minlevel);
   for (int l = minlevel; l <= maxlevel; l++) {
     if (l == minlevel)
       B.fill(l);
     else
-      B.prolong(0, l - 1, false);
-    B.tree_boundary(0, BK_HOM, l);
+      B.children(0, BK_HOM, l - 1);
+    B.boundary(0, BK_HOM, l);
     for (int i = 0; i < nrelax; i++) {
       TRY(B.relax(l));
-      B.tree_boundary(0, BK_HOM, l);
+      // after the last relax of a level: what the next level's initial
+      // guess reads
+      if (i + 1 < nrelax || l < maxlevel) B.boundary(0, BK_HOM, l);
     }
   }
   B.flush();
@@ -2055,9 +2258,20 @@ int cycle_kernels(bmg_tree* t, int nrelax, int minlevel, int maxlevel) {
   return BMG_OK;
 }
 
+// the boundary pass that ends a cycle, for a relax outside it
+template <typename T, int DIM>
+void pending_boundary(bmg_tree* t) {
+  if (t->da_level < 0) return;
+  Batcher<T, DIM> B(t, F<T>(t->da), F<T>(t->res), F<T>(t->tmp));
+  B.tree_boundary(0, BK_HOM, t->da_level);
+  B.flush();
+  t->da_level = -1;
+}
+
 template <typename T, int DIM>
 int mg_cycle(bmg_tree* t, int nrelax, int minlevel, int maxlevel) {
   TRY(coefficients<T, DIM>(t));
+  t->da_level = maxlevel;
   if (!t->use_graphs || t->prof) {
     TRY((cycle_kernels<T, DIM>(t, nrelax, minlevel, maxlevel)));
     tprof_collect(t);
@@ -2238,7 +2452,7 @@ int adapt_estimate(bmg_tree* t, const double* s, std::vector<double>& err_h) {
     int n = x.n_nonleaf[l];
     if (n)
       k_t_wavelet<DIM><<<nb_(n), kB, 0, t->stream>>>(x.rec_ring + (size_t)x.rec_off[l] * NR,
-                                                     x.rec_child0 + x.rec_off[l], n, s, err);
+                                                     x.rec_child0 + x.rec_off[l], n, s, x.box, err);
   }
   err_h.resize(x.nslot);
   hipError_t e = hipMemcpyAsync(err_h.data(), err, x.nslot * 8, hipMemcpyDeviceToHost, t->stream);
@@ -3075,6 +3289,8 @@ int adj_build(bmg_tree* t) {
   const int nrec = x.rec_off[D] + x.n_nonleaf[D] + x.n_prolong[D];
   std::vector<int> ring;
   TRY(download(ring, x.rec_ring, (size_t)nrec * NR));
+  for (int& v : ring)  // ghosts by their rule -> their slots
+    if (v < 0) v = ~v < nrules ? R[~v].ghost : -1;
   std::vector<int> pk;
   std::vector<bmgt::ProEnt> pv;
   pk.reserve((size_t)nrec * NCH * NCH);

@@ -59,6 +59,7 @@ __device__ __forceinline__ int seg_slot(const Segs& S, int s) {
 struct BoxRule {
   int ghost, src;
   int nterm;
+  int level;
   int side[3];
   int ti[3];  // index of the face value in the side's table
 };
@@ -82,8 +83,11 @@ __device__ __forceinline__ T bc_term(const BCT& bc, int bk, int side, int ti, do
   return (T)(D * v + (double)s);
 }
 
+// the value of a ghost cell from the rule's source (Delta as the host's
+// delta(): L0 times 2^-level)
 template <typename T>
-__device__ __forceinline__ void t_box_one(const BoxRule& q, T* __restrict__ f, const BCT& bc, int bk, double D) {
+__device__ __forceinline__ T t_box_value(const BoxRule& q, const T* f, const BCT& bc, int bk, double L0) {
+  const double D = L0 * (1. / (1 << q.level));
   T s = q.nterm ? f[q.src] : T(0);
   T v;
   if (q.nterm == 1)
@@ -95,17 +99,51 @@ __device__ __forceinline__ void t_box_one(const BoxRule& q, T* __restrict__ f, c
         bc_term<T>(bc, bk, q.side[2], q.ti[2], D, s) - T(2) * s;
   else
     v = (T)__builtin_nan("");
-  f[q.ghost] = v;
+  return v;
+}
+
+template <typename T>
+__device__ __forceinline__ void t_box_one(const BoxRule& q, T* __restrict__ f, const BCT& bc, int bk, double L0) {
+  f[q.ghost] = t_box_value<T>(q, f, bc, bk, L0);
 }
 
 template <typename T>
 __global__ __launch_bounds__(kB) void k_t_box(const BoxRule* __restrict__ R, int n, T* __restrict__ f, BCT bc, int bk,
-                                              double D) {
+                                              double L0) {
   int r = blockIdx.x * kB + threadIdx.x;
   if (r >= n) return;
   const BoxRule q = R[r];
-  t_box_one<T>(q, f, bc, bk, D);
+  t_box_one<T>(q, f, bc, bk, L0);
 }
+
+// An entry of the parent rings and of the colour lists' neighbour rows: a
+// slot, or ~r for the ghost cell that box rule r fills.  A reader either
+// takes the ghost's stored value (GhostStored, after the box pass of that
+// level) or evaluates the rule itself (GhostRule), which gives the value
+// that a box pass just before the read would have stored: the cycle does
+// the latter and runs no box pass at all.  A tree cycle is bound by the
+// number of its dependent launches (2-5 us each whatever their size), and
+// with the box pass of every level gone and only the values something reads
+// restricted and interpolated, a relax of the finest level of a quadtree of
+// levels 5-11 (225k leaves) takes 4 launches instead of 20: FP64 solve 44.6
+// -> 25.4 ms; octree of levels 4-8 (0.58M leaves), mixed, 26.3 -> 17.1 ms.
+template <typename T>
+struct GhostStored {
+  const T* f;
+  const BoxRule* box;
+  __device__ __forceinline__ T operator()(int v) const { return f[v >= 0 ? v : box[~v].ghost]; }
+};
+template <typename T>
+struct GhostRule {
+  const T* f;
+  const BoxRule* box;
+  const BCT& bc;
+  int bk;
+  double L0;
+  __device__ __forceinline__ T operator()(int v) const {
+    return v >= 0 ? f[v] : t_box_value<T>(box[~v], f, bc, bk, L0);
+  }
+};
 
 // restriction_average over the 2^dim children (child block in foreach_child
 // order) of each record
@@ -126,56 +164,103 @@ __global__ __launch_bounds__(kB) void k_t_restrict(const int* __restrict__ self,
   t_restrict_one<T, DIM>(f, self[r], child0[r]);
 }
 
-// bilinear (grid/multigrid-common.h:124-140) of the 2^dim children of a
-// record, in foreach_child order, from its 3^dim ring in src
+// the levels m0 .. m1 of a restriction in one launch: a workgroup takes the
+// records [r0, r1) of level m0 and everything below them, the finest level
+// first, with a barrier between levels.  The records of a level are in cache
+// order, so the children of a run of records are the run that `crec` (the
+// first child record of every record, per level) bounds.
+struct RestrictLevels {
+  int m0, m1, per_block;          // levels; records of level m0 per workgroup
+  int rec_off[kSeg], n[kSeg];     // records of each level
+  int crec_off[kSeg];             // its part of crec (n + 1 entries)
+};
+
 template <typename T, int DIM>
-__device__ __forceinline__ void t_bilinear_children(const int* __restrict__ g, const T* src, T* v) {
-  if (DIM == 2) {
-    T r[9];
-#pragma unroll
-    for (int m = 0; m < 9; m++) r[m] = src[g[m]];
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-      for (int b = 0; b < 2; b++) {
-        int cx = 2 * a - 1, cy = 2 * b - 1;
-        T c0 = r[4], c1 = r[(1 + cx) * 3 + 1], c2 = r[3 + 1 + cy], c3 = r[(1 + cx) * 3 + 1 + cy];
-        v[a * 2 + b] = (T(9) * c0 + T(3) * (c1 + c2) + c3) / T(16);
-      }
-  } else {
-#pragma unroll
-    for (int a = 0; a < 2; a++)
-#pragma unroll
-      for (int b = 0; b < 2; b++)
-#pragma unroll
-        for (int e = 0; e < 2; e++) {
-          int cx = 2 * a - 1, cy = 2 * b - 1, cz = 2 * e - 1;
-#define RG(x, y, z) src[g[((1 + (x)) * 3 + 1 + (y)) * 3 + 1 + (z)]]
-          T c000 = RG(0, 0, 0), c100 = RG(cx, 0, 0), c010 = RG(0, cy, 0), c001 = RG(0, 0, cz);
-          T c110 = RG(cx, cy, 0), c101 = RG(cx, 0, cz), c011 = RG(0, cy, cz), c111 = RG(cx, cy, cz);
-#undef RG
-          v[(a * 2 + b) * 2 + e] =
-              (T(27) * c000 + T(9) * (c100 + c010 + c001) + T(3) * (c110 + c101 + c011) + c111) / T(64);
-        }
+__global__ __launch_bounds__(kB) void k_t_restrict_tree(RestrictLevels L, const int* __restrict__ self,
+                                                        const int* __restrict__ child0, const int* __restrict__ crec,
+                                                        T* f) {
+  __shared__ int lo[kSeg], hi[kSeg];
+  if (threadIdx.x == 0) {
+    int a = min((int)blockIdx.x * L.per_block, L.n[L.m0]), b = min(a + L.per_block, L.n[L.m0]);
+    for (int m = L.m0;; m++) {
+      lo[m] = a;
+      hi[m] = b;
+      if (m == L.m1) break;
+      a = crec[L.crec_off[m] + a];
+      b = crec[L.crec_off[m] + b];
+    }
+  }
+  __syncthreads();
+  for (int m = L.m1; m >= L.m0; m--) {
+    for (int r = lo[m] + (int)threadIdx.x; r < hi[m]; r += kB)
+      t_restrict_one<T, DIM>(f, self[L.rec_off[m] + r], child0[L.rec_off[m] + r]);
+    __syncthreads();
   }
 }
 
-// bilinear into the 2^dim children of each record from its 3^dim ring
+// bilinear (grid/multigrid-common.h:124-140) of child m (foreach_child
+// order) of a record, from its 3^dim ring g read through `at`
+template <typename T, int DIM, typename L>
+__device__ __forceinline__ T t_bilinear_child(const int* __restrict__ g, int m, const L& at) {
+  if (DIM == 2) {
+    const int cx = 2 * (m >> 1) - 1, cy = 2 * (m & 1) - 1;
+    T c0 = at(g[4]), c1 = at(g[(1 + cx) * 3 + 1]), c2 = at(g[3 + 1 + cy]), c3 = at(g[(1 + cx) * 3 + 1 + cy]);
+    return (T(9) * c0 + T(3) * (c1 + c2) + c3) / T(16);
+  } else {
+    const int cx = 2 * (m >> 2) - 1, cy = 2 * ((m >> 1) & 1) - 1, cz = 2 * (m & 1) - 1;
+#define RG(x, y, z) at(g[((1 + (x)) * 3 + 1 + (y)) * 3 + 1 + (z)])
+    T c000 = RG(0, 0, 0), c100 = RG(cx, 0, 0), c010 = RG(0, cy, 0), c001 = RG(0, 0, cz);
+    T c110 = RG(cx, cy, 0), c101 = RG(cx, 0, cz), c011 = RG(0, cy, cz), c111 = RG(cx, cy, cz);
+#undef RG
+    return (T(27) * c000 + T(9) * (c100 + c010 + c001) + T(3) * (c110 + c101 + c011) + c111) / T(64);
+  }
+}
+
+// the 2^dim children of a record
+template <typename T, int DIM, typename L>
+__device__ __forceinline__ void t_bilinear_children(const int* __restrict__ g, const L& at, T* v) {
+#pragma unroll
+  for (int m = 0; m < (1 << DIM); m++) v[m] = t_bilinear_child<T, DIM>(g, m, at);
+}
+
+// bilinear into the 2^dim children of each record from its 3^dim ring, with
+// the ghosts stored in f
 template <typename T, int DIM>
-__device__ __forceinline__ void t_prolong_one(const int* __restrict__ g, int child0, T* f) {
+__device__ __forceinline__ void t_prolong_one(const int* __restrict__ g, int child0, T* f, const BoxRule* box) {
   T v[1 << DIM];
-  t_bilinear_children<T, DIM>(g, f, v);
+  t_bilinear_children<T, DIM>(g, GhostStored<T>{f, box}, v);
 #pragma unroll
   for (int m = 0; m < (1 << DIM); m++) f[child0 + m] = v[m];
 }
 
 template <typename T, int DIM>
 __global__ __launch_bounds__(kB) void k_t_prolong(const int* __restrict__ ring, const int* __restrict__ child0, int n,
-                                                  T* __restrict__ f) {
+                                                  T* __restrict__ f, const BoxRule* __restrict__ box) {
   int r = blockIdx.x * kB + threadIdx.x;
   if (r >= n) return;
   constexpr int NR = DIM == 2 ? 9 : 27;
-  t_prolong_one<T, DIM>(ring + (size_t)r * NR, child0[r], f);
+  t_prolong_one<T, DIM>(ring + (size_t)r * NR, child0[r], f, box);
+}
+
+// one child per thread: child `item % 2^dim` of record `item / 2^dim`, from
+// the records' rings with the ghosts' rules evaluated here.  The items are a
+// list (the halo cells of one dependency stage) or, with no list, all
+// children of n / 2^dim records.
+template <typename T, int DIM>
+__device__ __forceinline__ void t_child_one(int item, const int* __restrict__ ring, const int* __restrict__ child0,
+                                            T* f, const BoxRule* box, const BCT& bc, int bk, double L0) {
+  constexpr int NR = DIM == 2 ? 9 : 27;
+  const int r = item >> DIM, m = item & ((1 << DIM) - 1);
+  f[child0[r] + m] = t_bilinear_child<T, DIM>(ring + (size_t)r * NR, m, GhostRule<T>{f, box, bc, bk, L0});
+}
+
+template <typename T, int DIM>
+__global__ __launch_bounds__(kB) void k_t_children(const int* __restrict__ items, int n, const int* __restrict__ ring,
+                                                   const int* __restrict__ child0, T* f,
+                                                   const BoxRule* __restrict__ box, BCT bc, int bk, double L0) {
+  const int t = blockIdx.x * kB + threadIdx.x;
+  if (t >= n) return;
+  t_child_one<T, DIM>(items ? items[t] : t, ring, child0, f, box, bc, bk, L0);
 }
 
 // per-dimension coefficient pointers of relax (null = constant)
@@ -187,39 +272,40 @@ struct RelaxCoef {
   T lam_c;
 };
 
-// the value n/d of poisson.h:303-320 at slot gs (active index ai)
+// the value n/d of poisson.h:303-320 at slot gs; nb holds the cell's 2 dim
+// neighbours as slots or box rules (see GhostRule)
 template <typename T, int DIM>
-__device__ __forceinline__ T t_relax_value(const T* __restrict__ da, const T* __restrict__ res,
+__device__ __forceinline__ T t_relax_value(const GhostRule<T>& da, const T* __restrict__ res,
                                            const int* __restrict__ nb, const RelaxCoef<T>& k, int gs, T D2) {
   T n = -D2 * res[gs], d = -(k.lam ? k.lam[gs] : k.lam_c) * D2;
 #pragma unroll
   for (int c = 0; c < DIM; c++) {
     int lo = nb[2 * c], hi = nb[2 * c + 1];
-    T ah = k.alpha[c] ? k.alpha[c][hi] : k.alpha_c, al = k.alpha[c] ? k.alpha[c][gs] : k.alpha_c;
-    n += ah * da[hi] + al * da[lo];
+    T ah = k.alpha[c] ? k.alpha[c][hi >= 0 ? hi : da.box[~hi].ghost] : k.alpha_c;
+    T al = k.alpha[c] ? k.alpha[c][gs] : k.alpha_c;
+    n += ah * da(hi) + al * da(lo);
     d += ah + al;
   }
   return n / d;
 }
 
-// relaxation of the cells of foreach_level_or_leaf(l).  colour < 0: all
-// cells, value written to out (Jacobi's c); colour 0/1: in place, cells of
-// that colour only; 2: in place, every cell of the segments (lists of one
-// colour)
+// relaxation of the cells of foreach_level_or_leaf(l), segments of one colour
+// (their lists): in place, or the value to out (Jacobi's c).  A segment
+// without a list has its neighbours in the table nbr (slots only: the ghosts'
+// stored values).
 template <typename T, int DIM>
-__global__ __launch_bounds__(kB) void k_t_relax(Segs S, T* __restrict__ da, T* __restrict__ out,
-                                                const T* __restrict__ res, const int* __restrict__ nbr,
-                                                const uint8_t* __restrict__ colour, RelaxCoef<T> k, int sel) {
+__global__ __launch_bounds__(kB) void k_t_relax(Segs S, T* da, T* __restrict__ out, const T* __restrict__ res,
+                                                const int* __restrict__ nbr, const BoxRule* __restrict__ box, BCT bc,
+                                                double L0, RelaxCoef<T> k) {
   int s = seg_of(S);
   int gs = seg_slot(S, s);
   if (gs < 0) return;
   int ai = S.abase[s] + (gs - S.lvoff[s]);
-  if ((sel == 0 || sel == 1) && colour[ai] != sel) return;
   T D = (T)S.D[s];
   const int t = ((int)blockIdx.x - S.first_block[s]) * kB + (int)threadIdx.x;
   const int* nb = S.nbl[s] ? S.nbl[s] + (size_t)t * 2 * DIM : nbr + (size_t)ai * 2 * DIM;
-  T v = t_relax_value<T, DIM>(da, res, nb, k, gs, D * D);
-  if (sel < 0)
+  T v = t_relax_value<T, DIM>(GhostRule<T>{da, box, bc, BK_HOM, L0}, res, nb, k, gs, D * D);
+  if (out)
     out[gs] = v;
   else
     da[gs] = v;
@@ -529,14 +615,27 @@ __global__ void k_t_sum_final(const double* __restrict__ part, int np, double* _
 // workgroup, in order, with a barrier between them.  The operations and the
 // arithmetic are those of the standalone kernels above.
 
-enum { TOP_RESTRICT = 0, TOP_PROLONG = 1, TOP_BOX = 2, TOP_RELAX = 3, TOP_JACOBI = 4, TOP_FILL = 5 };
+// TOP_PROLONG, TOP_BOX: with the ghosts stored (the boundary pass of a field
+// that is handed on); TOP_CHILDREN (nonleaf records of a level), TOP_HALO (a
+// stage of halo cells), TOP_RELAX: the cycle's, with the ghosts' rules
+enum {
+  TOP_RESTRICT = 0,
+  TOP_PROLONG = 1,
+  TOP_BOX = 2,
+  TOP_RELAX = 3,
+  TOP_JACOBI = 4,
+  TOP_FILL = 5,
+  TOP_CHILDREN = 6,
+  TOP_HALO = 7
+};
 constexpr int kOpsBlock = 1024;
-constexpr int kMaxOps = 250;
+constexpr int kMaxOps = 200;
 
 struct TOp {
   unsigned char code, field;
-  signed char arg;  // prolong: halo; box: bc kind; relax: colour (-1: Jacobi value to tmp)
-  unsigned char level;
+  signed char arg;  // prolong: halo; box, children, halo: bc kind; relax: colour (-1: Jacobi value to tmp)
+  unsigned char level;  // halo: the finest level of the stage's cells
+  unsigned char stage;  // halo
 };
 
 struct TOps {
@@ -547,13 +646,15 @@ struct TOps {
 // per-level extents of the index tables
 struct TLevelInfo {
   int off, nA, abase, rec_off, n_nonleaf, n_prolong, box_off, box_n, leaf_off, leaf_n;
+  int col_off[2], col_n[2], lcol_off[2], lcol_n[2];  // colour lists: the level's cells, its leaves
 };
 
 template <typename T>
 struct TreeArgs {
   const TLevelInfo* lv;
-  const int *rec_self, *rec_child0, *rec_ring, *nbr, *lvl_leaves;
-  const uint8_t* colour;
+  const int *rec_self, *rec_child0, *rec_ring, *lvl_leaves, *col_list, *col_nbr;
+  const int *halo, *halo_end;  // halo cells by stage and level; per stage and level their end
+  int depth;
   const BoxRule* box;
   T* fld[3];  // fields an operation can name (da, res, tmp; or `a` alone)
   const T* res;
@@ -567,24 +668,26 @@ __device__ __forceinline__ void t_ops_cells(const TreeArgs<T>& A, const TOp& op)
   const int l = op.level;
   T* da = A.fld[0];
   for (int m = l; m >= 0; m--) {
-    const TLevelInfo L = A.lv[m];
-    const int n = m == l ? L.nA : L.leaf_n;
-    const double Dm = A.L0 * (1. / (1 << m));
-    for (int i = threadIdx.x; i < n; i += (int)blockDim.x) {
-      const int gs = m == l ? L.off + i : A.lvl_leaves[L.leaf_off + i];
-      const int ai = L.abase + (gs - L.off);
-      if (op.code == TOP_FILL) {
-        A.fld[op.field][gs] = T(0);
-      } else if (op.code == TOP_JACOBI) {
-        da[gs] = (da[gs] + T(2) * A.fld[2][gs]) / T(3);
-      } else {
-        if (op.arg >= 0 && A.colour[ai] != op.arg) continue;
-        const T D = (T)Dm;
-        T v = t_relax_value<T, DIM>(da, A.res, A.nbr + (size_t)ai * 2 * DIM, A.k, gs, D * D);
-        if (op.arg < 0)
-          A.fld[2][gs] = v;
+    const TLevelInfo& L = A.lv[m];
+    if (op.code == TOP_RELAX) {
+      const T Dm = (T)(A.L0 * (1. / (1 << m)));
+      for (int c = op.arg < 0 ? 0 : op.arg; c <= (op.arg < 0 ? 1 : op.arg); c++) {
+        const int o = m == l ? L.col_off[c] : L.lcol_off[c], n = m == l ? L.col_n[c] : L.lcol_n[c];
+        for (int i = threadIdx.x; i < n; i += (int)blockDim.x) {
+          const int gs = A.col_list[o + i];
+          const T v = t_relax_value<T, DIM>(GhostRule<T>{da, A.box, A.bc, BK_HOM, A.L0}, A.res,
+                                            A.col_nbr + (size_t)(o + i) * 2 * DIM, A.k, gs, Dm * Dm);
+          (op.arg < 0 ? A.fld[2] : da)[gs] = v;
+        }
+      }
+    } else {
+      const int n = m == l ? L.nA : L.leaf_n;
+      for (int i = threadIdx.x; i < n; i += (int)blockDim.x) {
+        const int gs = m == l ? L.off + i : A.lvl_leaves[L.leaf_off + i];
+        if (op.code == TOP_FILL)
+          A.fld[op.field][gs] = T(0);
         else
-          da[gs] = v;
+          da[gs] = (da[gs] + T(2) * A.fld[2][gs]) / T(3);
       }
     }
   }
@@ -606,15 +709,25 @@ __global__ __launch_bounds__(kOpsBlock) void k_t_ops(TOps P, TreeArgs<T> A) {
         const int r0 = L.rec_off + (op.arg ? L.n_nonleaf : 0);
         const int n = op.arg ? L.n_prolong : L.n_nonleaf;
         for (int r = threadIdx.x; r < n; r += (int)blockDim.x)
-          t_prolong_one<T, DIM>(A.rec_ring + (size_t)(r0 + r) * NR, A.rec_child0[r0 + r], f);
+          t_prolong_one<T, DIM>(A.rec_ring + (size_t)(r0 + r) * NR, A.rec_child0[r0 + r], f, A.box);
         break;
       }
       case TOP_BOX: {
-        const double D = A.L0 * (1. / (1 << op.level));
         for (int r = threadIdx.x; r < L.box_n; r += (int)blockDim.x) {
           const BoxRule q = A.box[L.box_off + r];
-          t_box_one<T>(q, f, A.bc, op.arg, D);
+          t_box_one<T>(q, f, A.bc, op.arg, A.L0);
         }
+        break;
+      }
+      case TOP_CHILDREN:
+        for (int i = threadIdx.x; i < L.n_nonleaf << DIM; i += (int)blockDim.x)
+          t_child_one<T, DIM>((L.rec_off << DIM) + i, A.rec_ring, A.rec_child0, f, A.box, A.bc, op.arg, A.L0);
+        break;
+      case TOP_HALO: {
+        const int i0 = op.stage ? A.halo_end[(op.stage - 1) * (A.depth + 1) + A.depth] : 0;
+        const int i1 = A.halo_end[op.stage * (A.depth + 1) + op.level];
+        for (int i = i0 + (int)threadIdx.x; i < i1; i += (int)blockDim.x)
+          t_child_one<T, DIM>(A.halo[i], A.rec_ring, A.rec_child0, f, A.box, A.bc, op.arg, A.L0);
         break;
       }
       default:
@@ -631,12 +744,13 @@ __global__ __launch_bounds__(kOpsBlock) void k_t_ops(TOps P, TreeArgs<T> A) {
 // parent's ring|
 template <int DIM>
 __global__ __launch_bounds__(kB) void k_t_wavelet(const int* __restrict__ ring, const int* __restrict__ child0, int n,
-                                                  const double* __restrict__ f, double* __restrict__ err) {
+                                                  const double* __restrict__ f, const BoxRule* __restrict__ box,
+                                                  double* __restrict__ err) {
   int r = blockIdx.x * kB + threadIdx.x;
   if (r >= n) return;
   constexpr int NR = DIM == 2 ? 9 : 27;
   double v[1 << DIM];
-  t_bilinear_children<double, DIM>(ring + (size_t)r * NR, f, v);
+  t_bilinear_children<double, DIM>(ring + (size_t)r * NR, GhostStored<double>{f, box}, v);
   const int c0 = child0[r];
 #pragma unroll
   for (int m = 0; m < (1 << DIM); m++) err[c0 + m] = fabs(f[c0 + m] - v[m]);
@@ -662,7 +776,7 @@ __global__ __launch_bounds__(kB) void k_t_refine_remap(const int* __restrict__ r
   if (r >= n) return;
   constexpr int NR = DIM == 2 ? 9 : 27;
   double v[1 << DIM];
-  t_bilinear_children<double, DIM>(ring + (size_t)r * NR, old, v);
+  t_bilinear_children<double, DIM>(ring + (size_t)r * NR, GhostStored<double>{old, nullptr}, v);
   const int c0 = child0[r];
 #pragma unroll
   for (int m = 0; m < (1 << DIM); m++) out[c0 + m] = v[m];

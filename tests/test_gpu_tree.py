@@ -214,3 +214,47 @@ def test_tree_project_bitexact(dim, depth, dt):
     so2 = o.project(uo, dt=dt)
     assert sg2["i"] == so2["i"] and sg2["resa"] == so2["resa"]
     assert np.array_equal(ud.cpu().numpy(), uo)
+
+
+@pytest.mark.parametrize("smoother", ["jacobi", "rbgs"])
+@pytest.mark.parametrize("dim,depth,minlevel", [(2, 7, 3), (2, 8, 1), (3, 5, 2)])
+def test_cycle_launch_shapes_bitexact(dim, depth, minlevel, smoother, monkeypatch):
+    """The cycle's operations run batched in one workgroup, as launches of
+    their own (the several-level restriction among them), or mixed: every
+    split gives the oracle's values, on a tree with leaves from level 1 on
+    and several halo stages, for cycles from each coarsest level."""
+    o = OracleTree(dim, 1.0, (0.0, 0.0, 0.0))
+    o.set_smoother(smoother)
+    tree_cases.spheres_problem(o, depth, 11, nspheres=3, minlevel=minlevel)
+    o.restriction_alpha_lambda()
+    o.residual()
+    want = []
+    for m in (0, 1, minlevel, depth - 1):
+        o.mg_cycle(3, m, depth)
+        want.append(o.residual())
+    for small_op in ("1", "200", "1000000"):
+        print("launch shapes", dim, depth, minlevel, smoother, small_op, flush=True)
+        monkeypatch.setenv("BMG_TREE_SMALL_OP", small_op)
+        g = bmg.Tree(dim, 1.0, (0.0, 0.0, 0.0), smoother=smoother)
+        tree_cases.spheres_problem(g, depth, 11, nspheres=3, minlevel=minlevel)
+        g.restriction_alpha_lambda()
+        g.residual()
+        for m, r in zip((0, 1, minlevel, depth - 1), want):
+            g.mg_cycle(3, m, depth)
+            assert g.residual() == r
+        assert np.array_equal(g.get_a(), o.get_a())
+
+
+@pytest.mark.parametrize("smoother", ["jacobi", "rbgs"])
+def test_relax_after_cycle_sees_its_boundary(smoother):
+    """relax() on the finest level right after a cycle of that level alone
+    equals one more relax in the cycle."""
+    t = [bmg.Tree(2, 1.0, (0.0, 0.0, 0.0), smoother=smoother) for _ in range(2)]
+    for g in t:
+        tree_cases.spheres_problem(g, 7, 11, nspheres=3)
+        g.residual()
+    print("relax after cycle", smoother, flush=True)
+    t[0].mg_cycle(3, 7, 7)
+    t[0].relax(7)
+    t[1].mg_cycle(4, 7, 7)
+    assert np.array_equal(t[0].get_da(), t[1].get_da())
