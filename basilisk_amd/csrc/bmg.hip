@@ -18,6 +18,7 @@
 
 #include "../../include/bmg.h"
 #include "bmg_internal.h"
+#include "bmg_block_kernels.h"
 #include "bmg_embed_kernels.h"
 #include "bmg_kernels.h"
 #include "bmg_visc_kernels.h"
@@ -641,7 +642,8 @@ int emb_check(const bmg_grid* g, int minlevel) {
 // relax kernel of a level: two-launch in-place red-black (tiny levels),
 // one-launch fused red-black, single-pass streaming red-black (3D,
 // n >= 128) or Jacobi
-enum { RK_INPLACE_RB, RK_FUSED_RB, RK_STREAM_RB, RK_STREAM2_RB, RK_STREAM3_RB, RK_PAIR_RB, RK_JACOBI, RK_GS, RK_EMBED };
+enum { RK_INPLACE_RB, RK_FUSED_RB, RK_STREAM_RB, RK_STREAM2_RB, RK_STREAM3_RB, RK_PAIR_RB, RK_TILE_RB, RK_JACOBI, RK_GS,
+       RK_EMBED };
 
 // a cell-count threshold with an environment override (tuning knob)
 size_t size_knob(const char* name, size_t dflt) {
@@ -695,17 +697,38 @@ int level_kernel(const bmg_grid* g, int l) {
       ((g->rb_override != RK_STREAM_RB && g->rb_override != RK_STREAM2_RB && g->rb_override != RK_STREAM3_RB) ||
        (g->rb_override == RK_STREAM3_RB ? stream3 : DIM == 3 && g->L[l].n >= 128)))
     return g->rb_override;
-  // measured at 256^3: the single-pass column-streamed kernel reads each
-  // operand once and beats the two-launch in-place kernel, which is the
-  // fastest on every other level now that the cycle replays as a graph (the
-  // one-launch fused kernel, which recomputes red neighbours, only paid off
-  // while launches were issued one by one; BMG_FUSED_MIN brings it back for
-  // levels of at least that many cells, below BMG_INPLACE_MIN)
+  // the single-pass column-streamed kernel reads each operand once; the
+  // levels it does not take (2D, 3D below 128^3, periodic) run several
+  // half-sweeps per launch from LDS (k_rb_tile), in the cycle; the one-launch
+  // fused kernel, which recomputes red neighbours, only paid off while
+  // launches were issued one by one (BMG_FUSED_MIN brings it back for levels
+  // of at least that many cells, below BMG_INPLACE_MIN)
   if (stream3 && g->rb_override < 0) return RK_STREAM3_RB;
   const size_t nc = g->L[l].ncell;
   if (nc >= size_knob("BMG_FUSED_MIN", ~(size_t)0) && nc < size_knob("BMG_INPLACE_MIN", 1u << 20))
     return RK_FUSED_RB;
-  return RK_INPLACE_RB;
+  const bool tile = DIM == 2 || (DIM == 3 && (size_t)g->L[l].n <= size_knob("BMG_TILE_MAX3", 64));
+  return tile && g->rb_override < 0 && g->L[l].n >= 16 ? RK_TILE_RB : RK_INPLACE_RB;
+}
+
+// k_rb_tile on an n^DIM level: the region (a variant of the kernel) and the
+// sweeps per launch.  2D: up to 4 sweeps per launch (two launches of 2 take
+// 39 instead of 28 us at 1024^2, FP64), on the smallest region that leaves
+// the level at most about two workgroups per CU.  3D: 2 sweeps on 16^3 cells
+// (one sweep per launch: 15 instead of 11 us for two on 32^3 and 64^3, FP32;
+// the in-place kernel 16 us and 6 us of prolongation); at 128^3 recomputing
+// the halos costs more than the launches (25 against 24 us a sweep).
+template <int DIM>
+int tile_variant(int n) {
+  if (DIM == 2) return n <= 256 ? 0 : n <= 512 ? 1 : 2;
+  return n <= 64 ? 0 : 1;
+}
+
+template <int DIM>
+int tile_sweeps(int n) {
+  const int dflt = DIM == 2 ? 4 : n <= 64 ? 2 : 1;
+  const size_t v = size_knob("BMG_TILE_SWEEPS", dflt);
+  return v >= 1 && v <= (DIM == 2 ? 4u : 2u) ? (int)v : dflt;
 }
 
 // planes per workgroup of the streaming kernels (BMG_STREAM_CHUNK overrides,
@@ -719,10 +742,20 @@ int stream_chunk(int n) {
 }
 
 
+bool coarse_in_lds(const bmg_grid* g) {
+  return g->smoother == BMG_RELAX_RBGS && g->dim >= 2 && g->rb_override < 0;
+}
+
 // largest level that the single-workgroup coarse kernel takes (at most 4096
 // cells; BMG_COARSE_TOP overrides within that limit)
 int coarse_top(const bmg_grid* g) {
-  int top = g->dim == 3 ? 3 : g->dim == 2 ? 5 : 10;
+  // levels of 512-1024 cells; red-black in 3D (k_coarse_rb, on chip) the
+  // 16^3 level too, unless its registers do not suffice: 12 us for its
+  // sweeps in this kernel against two launches of 10 us by tiles and the
+  // restriction's own (64^2: 8 us against 5 and 2)
+  const bool lds = coarse_in_lds(g), few = g->precision == BMG_FP64 && g->alpha_field;
+  int top = g->dim == 3 ? (lds && !few ? 4 : 3) : g->dim == 2 ? 5 : 10;
+  if (lds) return std::min(top, g->depth);
   if (const char* e = getenv("BMG_COARSE_TOP")) {
     int v = atoi(e), lim = g->dim == 3 ? 4 : g->dim == 2 ? 6 : 12;
     if (v >= 0 && v <= lim) top = v;
@@ -993,10 +1026,60 @@ int coarse_block(bmg_grid* g, int nrelax, int minlevel, int top) {
   A.jacobi = g->smoother == BMG_RELAX_JACOBI;
   A.gs = g->smoother == BMG_RELAX_GS;
   ProfScope ps(g, PROF_RELAX_COARSE);
+  if constexpr (DIM >= 2) {
+    if (coarse_in_lds(g)) {
+      // a thread per block of the largest level
+      const size_t blocks = g->L[top].ncell >> DIM;
+      const dim3 nt((unsigned)std::max<size_t>(64, blocks));
+      if (g->alpha_field) hipLaunchKernelGGL((k_coarse_rb<DIM, T, true>), dim3(1), nt, 0, g->stream, A);
+      else hipLaunchKernelGGL((k_coarse_rb<DIM, T, false>), dim3(1), nt, 0, g->stream, A);
+      return check_launch();
+    }
+  }
   // threads of the workgroup (BMG_COARSE_BLOCK: a multiple of 64 up to 1024)
   size_t nt = size_knob("BMG_COARSE_BLOCK", 1024);
   if (nt > 1024 || nt % 64) nt = 1024;
   hipLaunchKernelGGL((k_coarse_cycle<DIM, T>), dim3(1), dim3((unsigned)nt), 0, g->stream, A);
+  return check_launch();
+}
+
+// ns sweeps of level l by tiles: da[src], or the bilinear initial guess when
+// src < 0, into da[dst]; with correct, a += da as well
+template <int DIM, typename T>
+int tile_sweep(bmg_grid* g, int l, int ns, int src, int dst, bool correct) {
+  Level& lv = g->L[l];
+  const Geo<DIM> geo{lv.n, lv.log2n};
+  const BCH bc = level_bc<DIM>(g, l), bcc = level_bc<DIM>(g, l - 1);
+  const Coef<T> k = level_coef<T>(g, l);
+  const double D = delta(g, l);
+  auto go = [&](auto kern, int b0, int b1, int b2) {
+    const int R[3] = {2 * b0, 2 * b1, 2 * b2}, nt = b0 * b1 * b2;
+    TileArgs A{};
+    A.ns = ns;
+    size_t nb = 1;
+    for (int d = 0; d < DIM; d++) {
+      const bool whole = R[d] >= lv.n && !bc.periodic[d];
+      A.halo[d] = whole ? 0 : 2 * ns;
+      A.tile[d] = whole ? lv.n : R[d] - 4 * ns;
+      A.ntile[d] = (lv.n + A.tile[d] - 1) / A.tile[d];
+      nb *= (size_t)A.ntile[d];
+    }
+    for (int d = DIM; d < 3; d++) A.ntile[d] = A.tile[d] = 1;
+    hipLaunchKernelGGL(kern, dim3((unsigned)nb), dim3(nt), 0, g->stream, src < 0 ? nullptr : (const T*)lv.da[src],
+                       src < 0 ? (const T*)g->L[l - 1].da[0] : nullptr, (T*)lv.da[dst], correct ? g->a : nullptr,
+                       (const T*)lv.res, k, geo, bc, bcc, (T)(D * D), A);
+  };
+  ProfScope ps(g, l == g->depth ? PROF_RELAX_FINE : PROF_RELAX_COARSE);
+  const bool af = k.lo[0] != nullptr;
+  [[maybe_unused]] const int v = tile_variant<DIM>(lv.n);
+  if constexpr (DIM == 2) {
+    if (v == 0) af ? go(k_rb_tile<2, T, true, 16, 16, 1>, 16, 16, 1) : go(k_rb_tile<2, T, false, 16, 16, 1>, 16, 16, 1);
+    else if (v == 1) af ? go(k_rb_tile<2, T, true, 24, 24, 1>, 24, 24, 1)
+                        : go(k_rb_tile<2, T, false, 24, 24, 1>, 24, 24, 1);
+    else af ? go(k_rb_tile<2, T, true, 32, 32, 1>, 32, 32, 1) : go(k_rb_tile<2, T, false, 32, 32, 1>, 32, 32, 1);
+  } else if constexpr (DIM == 3) {
+    af ? go(k_rb_tile<3, T, true, 8, 8, 8>, 8, 8, 8) : go(k_rb_tile<3, T, false, 8, 8, 8>, 8, 8, 8);
+  }
   return check_launch();
 }
 
@@ -1034,14 +1117,34 @@ int mg_cycle_t(bmg_grid* g, int nrelax, int minlevel, int maxlevel, bool defer) 
   TRY(check_launch());
   // the coarse levels in one workgroup; they end in da[0]
   if (use_block) TRY((coarse_block<DIM, T>(g, nrelax, minlevel, top)));
+  bool corrected = false;
   for (int l = use_block ? top + 1 : minlevel; l <= maxlevel; l++) {
     Level& lv = g->L[l];
     // ping-pong sweeps start in da[flips & 1] so that they end in da[0]
     // (a two-sweep launch flips the buffers once)
     const int rk = level_kernel<DIM>(g, l);
+    if (rk == RK_TILE_RB && nrelax > 0 && l > 0) {
+      // launches ping-pong between the buffers and end in da[0]; the first
+      // one interpolates the initial guess, the last one of a cycle that
+      // corrects by itself adds the correction
+      const int nl = (nrelax + tile_sweeps<DIM>(lv.n) - 1) / tile_sweeps<DIM>(lv.n);
+      const bool own = l == g->depth && !(defer && maxlevel == g->depth);
+      if (l == minlevel)
+        hipLaunchKernelGGL((k_fill<T>), dim3(nblocks(lv.ncell)), dim3(kBlock), 0, g->stream, (T*)lv.da[nl & 1],
+                           lv.ncell, T(0));
+      int left = nrelax;
+      for (int j = 0; j < nl; j++) {
+        const int ns = (left + nl - j - 1) / (nl - j);
+        left -= ns;
+        TRY((tile_sweep<DIM, T>(g, l, ns, j == 0 && l > minlevel ? -1 : (nl - j) & 1, (nl - 1 - j) & 1,
+                                own && j == nl - 1)));
+      }
+      corrected = own;
+      continue;
+    }
     const bool two = use_sweep2<DIM, T>(g, l);
     const int flips = two ? nrelax - nrelax / 2 : nrelax;
-    const bool inplace = rk == RK_INPLACE_RB || rk == RK_PAIR_RB ||
+    const bool inplace = rk == RK_INPLACE_RB || rk == RK_TILE_RB || rk == RK_PAIR_RB ||
                          (rk == RK_EMBED && g->smoother == BMG_RELAX_RBGS);
     int dst = inplace ? 0 : (flips & 1);
     if (l == minlevel) {
@@ -1090,7 +1193,7 @@ int mg_cycle_t(bmg_grid* g, int nrelax, int minlevel, int maxlevel, bool defer) 
     g->pending_correct = true;
     return BMG_OK;
   }
-  {
+  if (!corrected) {
     ProfScope ps(g, PROF_CORRECT);
     hipLaunchKernelGGL((k_correct<T>), dim3(nblocks(lf.ncell)), dim3(kBlock), 0, g->stream, g->a,
                        (const T*)lf.da[0], lf.ncell);

@@ -499,8 +499,9 @@ __device__ __forceinline__ T coarse_at(const T* __restrict__ f, const Geo<DIM>& 
 // index contributions of the two coarse cells along one dimension of the
 // bilinear stencil: the parent p and its neighbour p+o (o = -1 or +1),
 // mapped like a ghost cell (wrapped, or the parent itself with sign sigma)
-template <int DIM, typename T>
-__device__ __forceinline__ void axis_pair(const Geo<DIM>& gc, const BCH& bc, int d, int p, int o, idx_t& off0,
+// (the geometry gives n and the strides)
+template <int DIM, typename T, typename G>
+__device__ __forceinline__ void axis_pair(const G& gc, const BCH& bc, int d, int p, int o, idx_t& off0,
                                           idx_t& off1, T& sg, bool& gh) {
   const idx_t s = gc.stride(d);
   const int q = p + o;
@@ -532,8 +533,8 @@ __device__ __forceinline__ T corner3(T v, T sx, T sy, T sz, bool gx, bool gy, bo
 
 // bilinear value at fine cell c from the coarse level,
 // grid/multigrid-common.h:124-140, child offsets grid/multigrid.h:175-188
-template <int DIM, typename T>
-__device__ __forceinline__ T bilinear_at(const T* __restrict__ coarse, const Geo<DIM>& gc, const BCH& bcc,
+template <int DIM, typename T, typename G>
+__device__ __forceinline__ T bilinear_at(const T* __restrict__ coarse, const G& gc, const BCH& bcc,
                                          const int c[3]) {
   idx_t x0, x1, y0 = 0, y1 = 0, z0 = 0, z1 = 0;
   T sx, sy = T(1), sz = T(1);
