@@ -2753,6 +2753,26 @@ struct Visc {
     A.y0 = g->X0[1];
     return A;
   }
+  // the correction's boundary conditions of level l, per component
+  ViscBC homogeneous(int l) const {
+    ViscBC B;
+    memset(&B, 0, sizeof B);
+    bool anyp = false;
+    for (int d = 0; d < DIM; d++) anyp |= g->periodic[d] != 0;
+    for (int c = 0; c < DIM; c++) {
+      for (int d = 0; d < DIM; d++) B.bc[c].periodic[d] = g->periodic[d];
+      for (int b = 0; b < 6; b++) B.bc[c].sigma[b] = l == 0 && anyp ? 1 : sig[c][b];
+    }
+    return B;
+  }
+  Comp3 comps(double* const* in, double* const* out) const {
+    Comp3 A;
+    for (int c = 0; c < 3; c++) {
+      A.in[c] = c < DIM ? in[c] : nullptr;
+      A.out[c] = c < DIM ? out[c] : nullptr;
+    }
+    return A;
+  }
   double* const* lv(int l, int slot) const { return &g->visc[(size_t)l * kViscSlots + slot]; }
 
   // restriction ({mu, rho}) (viscosity.h:173-175)
@@ -2777,9 +2797,11 @@ struct Visc {
   int residual(double* maxres, unsigned long long* nans) {
     const Level& lf = g->L[g->depth];
     Geo<DIM> geo{lf.n, lf.log2n};
-    hipLaunchKernelGGL(k_stat_reset, dim3(1), dim3(64), 0, g->stream, g->stat);
-    hipLaunchKernelGGL((k_visc_residual<DIM>), dim3(std::min(nblocks(lf.ncell), 8192u)), dim3(kBlock), 0, g->stream,
-                       args(g->depth, u, lv(g->depth, VS_RES), g->visc_r), geo, g->stat);
+    // (g->part holds a partial per kBlock cells)
+    const unsigned nb = nblocks(lf.ncell);
+    hipLaunchKernelGGL((k_visc_residual<DIM>), dim3(nb), dim3(kBlock), 0, g->stream,
+                       args(g->depth, u, lv(g->depth, VS_RES), g->visc_r), geo, g->part);
+    hipLaunchKernelGGL(k_reduce_stat, dim3(1), dim3(1024), 0, g->stream, g->part, (int)nb, g->stat);
     TRY(check_launch());
     Stat st;
     HIPCHECK(hipMemcpyAsync(&st, g->stat, sizeof st, hipMemcpyDeviceToHost, g->stream));
@@ -2811,31 +2833,37 @@ struct Visc {
   // grid's smoother: red-black (default) or the reference's JACOBI variant
   int cycle(int nrelax) {
     const int D = g->depth;
-    for (int l = D - 1; l >= 0; l--) {
+    // red-black: the levels up to 8^3 or 32^2 in one workgroup
+    const int top = g->smoother == BMG_RELAX_RBGS ? std::min(D, DIM == 3 ? 3 : 5) : -1;
+    static_assert(kViscCoarse > 5 && sizeof(ViscCoarse) <= 4096, "kernel argument block");
+    for (int l = D - 1; l >= std::max(top, 0); l--) {
       Geo<DIM> gc{g->L[l].n, g->L[l].log2n};
-      for (int c = 0; c < DIM; c++)
-        hipLaunchKernelGGL((k_restrict<DIM, double>), dim3(nblocks(g->L[l].ncell)), dim3(kBlock), 0, g->stream,
-                           vbuf(g, l + 1, VS_RES + c), vbuf(g, l, VS_RES + c), gc);
+      hipLaunchKernelGGL((k_visc_restrict<DIM>), dim3(nblocks(g->L[l].ncell), DIM), dim3(kBlock), 0, g->stream,
+                         comps(lv(l + 1, VS_RES), lv(l, VS_RES)), gc);
     }
-    for (int l = 0; l <= D; l++) {
+    if (top >= 0) {
+      ViscCoarse A;
+      memset((void*)&A, 0, sizeof A);
+      for (int l = 0; l <= top; l++) {
+        A.L[l] = args(l, lv(l, VS_DA), lv(l, VS_DN), lv(l, VS_RES));
+        A.bc[l] = homogeneous(l);
+      }
+      A.top = top;
+      A.nrelax = nrelax;
+      hipLaunchKernelGGL((k_visc_coarse<DIM>), dim3(1), dim3(kViscThreads<DIM>), 0, g->stream, A);
+    }
+    for (int l = top + 1; l <= D; l++) {
       const Level& lv_ = g->L[l];
       Geo<DIM> gf{lv_.n, lv_.log2n};
-      for (int c = 0; c < DIM; c++) {
-        if (l == 0) {
+      if (l == 0) {
+        for (int c = 0; c < DIM; c++)
           hipLaunchKernelGGL((k_fill<double>), dim3(nblocks(lv_.ncell)), dim3(kBlock), 0, g->stream,
                              vbuf(g, l, VS_DA + c), lv_.ncell, 0.);
-        } else {
-          BCH bcc;
-          memset(&bcc, 0, sizeof bcc);
-          bool anyp = false;
-          for (int d = 0; d < 3; d++) {
-            bcc.periodic[d] = d < DIM ? g->periodic[d] : 0;
-            anyp |= bcc.periodic[d] != 0;
-          }
-          for (int b = 0; b < 6; b++) bcc.sigma[b] = (l - 1 == 0 && anyp) ? 1 : sig[c][b];
-          hipLaunchKernelGGL((k_prolong<DIM, double>), dim3(nblocks(lv_.ncell)), dim3(kBlock), 0, g->stream,
-                             vbuf(g, l - 1, VS_DA + c), vbuf(g, l, VS_DA + c), gf, bcc);
-        }
+      } else {
+        const Level& lc = g->L[l - 1];
+        Geo<DIM> gc{lc.n, lc.log2n};
+        hipLaunchKernelGGL((k_visc_prolong<DIM>), dim3(nblocks(lc.ncell), DIM), dim3(kBlock), 0, g->stream,
+                           comps(lv(l - 1, VS_DA), lv(l, VS_DA)), gc, homogeneous(l - 1));
       }
       // passes per sweep: Jacobi one (colour -1), Gauss-Seidel one (the
       // single cell of level 0 as colour 0), red-black two
@@ -2867,9 +2895,7 @@ struct Visc {
         }
     }
     const size_t n = g->L[D].ncell;
-    for (int c = 0; c < DIM; c++)
-      hipLaunchKernelGGL((k_correct<double>), dim3(nblocks(n)), dim3(kBlock), 0, g->stream, u[c],
-                         (const double*)vbuf(g, D, VS_DA + c), n);
+    hipLaunchKernelGGL(k_visc_correct, dim3(nblocks(n), DIM), dim3(kBlock), 0, g->stream, comps(lv(D, VS_DA), u), n);
     return check_launch();
   }
 

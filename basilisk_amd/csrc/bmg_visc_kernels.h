@@ -30,7 +30,7 @@
 
 #include <hip/hip_runtime.h>
 
-#include "bmg_kernels.h"
+#include "bmg_block_kernels.h"
 
 namespace bmg {
 
@@ -256,13 +256,11 @@ __global__ __launch_bounds__(kBlock) void k_visc_jacobi(ViscArgs A, Geo<DIM> g) 
 }
 
 // one red-black pass: the cells whose i+j+k has the parity `colour` take w,
-// read from the pass input, the others are copied.  One thread per pair of
+// read from the pass input, the others are copied.  One thread per pair t of
 // cells along the last dimension (one of each parity, so no wave diverges);
 // levels with n >= 2.
 template <int DIM>
-__global__ __launch_bounds__(kBlock) void k_visc_rb(ViscArgs A, Geo<DIM> g, int colour) {
-  const idx_t t = logical_block() * kBlock + threadIdx.x;
-  if (t >= g.ncell() / 2) return;
+__device__ __forceinline__ void visc_rb_pair(const ViscArgs& A, const Geo<DIM>& g, idx_t t, int colour) {
   const idx_t pair = 2 * t;  // the pair's first cell (k even)
   int x[3];
   g.decode(pair, x);
@@ -277,6 +275,13 @@ __global__ __launch_bounds__(kBlock) void k_visc_rb(ViscArgs A, Geo<DIM> g, int 
     A.out[c][idx] = w[c];
     A.out[c][other] = A.u[c][other];
   }
+}
+
+template <int DIM>
+__global__ __launch_bounds__(kBlock) void k_visc_rb(ViscArgs A, Geo<DIM> g, int colour) {
+  const idx_t t = logical_block() * kBlock + threadIdx.x;
+  if (t >= g.ncell() / 2) return;
+  visc_rb_pair<DIM>(A, g, t, colour);
 }
 
 // The Gauss-Seidel sweep: a cell reads the new values of the cells before
@@ -334,8 +339,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_gs_plane(ViscArgs A, Geo<DIM> g
 
 // the single cell of level 0: either parity, the same arithmetic
 template <int DIM>
-__global__ void k_visc_one(ViscArgs A, Geo<DIM> g, int colour) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__device__ __forceinline__ void visc_one(const ViscArgs& A, const Geo<DIM>& g, int colour) {
   int x[3] = {0, 0, 0};
   double w[3];
   visc_target<DIM>(A, g, 0, x, w);
@@ -346,14 +350,157 @@ __global__ void k_visc_one(ViscArgs A, Geo<DIM> g, int colour) {
   }
 }
 
+template <int DIM>
+__global__ void k_visc_one(ViscArgs A, Geo<DIM> g, int colour) {
+  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  visc_one<DIM>(A, g, colour);
+}
+
+// --- the passes around the sweeps, every component in one launch ----------
+// (blockIdx.y: the component)
+// One launch instead of one per component: prolongation, restriction and
+// correction of a cycle at 128^3 92 + 47 + 28 -> 32 + 18 + 26 us.
+struct Comp3 {
+  const double* in[3];
+  double* out[3];
+};
+
+template <int DIM>
+__device__ __forceinline__ double visc_mean(const double* __restrict__ fine, const Geo<DIM>& gc, idx_t idx) {
+  int c[3];
+  gc.decode(idx, c);
+  const Geo<DIM> gf{gc.n * 2, gc.log2n + 1};
+  const int f[3] = {2 * c[0], 2 * c[1], 2 * c[2]};
+  const idx_t b = gf.index(f);
+  double sum = 0.;
+#pragma unroll
+  for (int m = 0; m < (1 << (DIM - 1)); m++) {
+    const idx_t q = b + (DIM == 3 ? (idx_t)(m >> 1) * gf.stride(0) + (idx_t)(m & 1) * gf.stride(1)
+                                  : (idx_t)m * gf.stride(0));
+    sum += fine[q];
+    sum += fine[q + 1];
+  }
+  return sum / (double)(1 << DIM);
+}
+
+template <int DIM>
+__global__ __launch_bounds__(kBlock) void k_visc_restrict(Comp3 A, Geo<DIM> gc) {
+  const idx_t idx = logical_block() * kBlock + threadIdx.x;
+  const int c = blockIdx.y;
+  if (idx < gc.ncell()) A.out[c][idx] = visc_mean<DIM>(A.in[c], gc, idx);
+}
+
+// the initial guess: the 2^DIM children of coarse cell idx
+struct ViscBC {
+  BCH bc[3];  // of the coarse level, per component
+};
+
+template <int DIM>
+__device__ __forceinline__ void visc_children(const double* __restrict__ coarse, double* __restrict__ fine,
+                                              const Geo<DIM>& gc, const BCH& bc, idx_t idx) {
+  int c[3];
+  gc.decode(idx, c);
+  double v[1 << DIM];
+  bilinear_block<DIM, double>(c, gc.n, bc, [&](const int* q) { return coarse[gc.index(q)]; }, v);
+  const Geo<DIM> gf{gc.n * 2, gc.log2n + 1};
+  const int f[3] = {2 * c[0], 2 * c[1], 2 * c[2]};
+  const idx_t b = gf.index(f);
+#pragma unroll
+  for (int m = 0; m < (1 << (DIM - 1)); m++) {
+    const idx_t q = b + (DIM == 3 ? (idx_t)(m >> 1) * gf.stride(0) + (idx_t)(m & 1) * gf.stride(1)
+                                  : (idx_t)m * gf.stride(0));
+    *reinterpret_cast<double2*>(fine + q) = make_double2(v[2 * m], v[2 * m + 1]);
+  }
+}
+
+template <int DIM>
+__global__ __launch_bounds__(kBlock) void k_visc_prolong(Comp3 A, Geo<DIM> gc, ViscBC B) {
+  const idx_t idx = logical_block() * kBlock + threadIdx.x;
+  const int c = blockIdx.y;
+  if (idx < gc.ncell()) visc_children<DIM>(A.in[c], A.out[c], gc, B.bc[c], idx);
+}
+
+// u += da
+__global__ __launch_bounds__(kBlock) void k_visc_correct(Comp3 A, size_t n) {
+  const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
+  const int c = blockIdx.y;
+  if (i < n) A.out[c][i] += A.in[c][i];
+}
+
+// the levels 0..top of a red-black cycle (at most 1024 cells, 8^3 or 32^2) in
+// one workgroup: the restriction of res from level top, then per level the
+// zero or bilinear initial guess and nrelax sweeps, a pass per colour from
+// one buffer to the other (an even number, so that they end in u).  A pass
+// is as long here as the 4-5 us of its own launch at 8^3 and shorter below
+// (32^2: 2 us); what goes is the launches around the passes, and the host
+// stays ahead of the device.  One level more in 3D: 18.8 instead of 16.3 ms
+// for 31 cycles at 128^3; one less: the same.
+constexpr int kViscCoarse = 6;
+template <int DIM>
+constexpr int kViscThreads = DIM == 3 ? 256 : 512;
+
+struct ViscCoarse {
+  ViscArgs L[kViscCoarse];  // u: da, out: the other buffer, r: res
+  ViscBC bc[kViscCoarse];   // of each level
+  int top, nrelax;
+};
+
+template <int DIM>
+__global__ __launch_bounds__(kViscThreads<DIM>) void k_visc_coarse(ViscCoarse A) {
+  const idx_t t = threadIdx.x;
+  for (int l = A.top - 1; l >= 0; l--) {
+    const Geo<DIM> gc{1 << l, l};
+#pragma unroll
+    for (int c = 0; c < DIM; c++)
+      for (idx_t i = t; i < gc.ncell(); i += kViscThreads<DIM>)
+        const_cast<double*>(A.L[l].r[c])[i] = visc_mean<DIM>(A.L[l + 1].r[c], gc, i);
+    __syncthreads();
+  }
+  for (int l = 0; l <= A.top; l++) {
+    const Geo<DIM> g{1 << l, l};
+    ViscArgs V = A.L[l];
+#pragma unroll
+    for (int c = 0; c < DIM; c++) {
+      double* u = const_cast<double*>(V.u[c]);
+      if (l == 0) {
+        if (t == 0) u[0] = 0.;
+      } else {
+        const Geo<DIM> gc{1 << (l - 1), l - 1};
+        for (idx_t i = t; i < gc.ncell(); i += kViscThreads<DIM>)
+          visc_children<DIM>(A.L[l - 1].u[c], u, gc, A.bc[l - 1].bc[c], i);
+      }
+    }
+    __syncthreads();
+    for (int it = 0; it < A.nrelax; it++)
+      for (int col = 0; col < 2; col++) {
+        if (l == 0) {
+          if (t == 0) visc_one<DIM>(V, g, col);
+        } else {
+          for (idx_t i = t; i < g.ncell() / 2; i += kViscThreads<DIM>) visc_rb_pair<DIM>(V, g, i, col);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < DIM; c++) {
+          double* u = const_cast<double*>(V.u[c]);
+          V.u[c] = V.out[c];
+          V.out[c] = u;
+        }
+      }
+  }
+}
+
 // residual_viscosity on the finest level: res = r - u + dt/rho S / D^2,
 // max |res| over the components to st (NaN counted)
-// (a grid-stride loop over a capped grid: one atomic max per block)
+// (per block partials, which k_reduce_stat folds, instead of 8192 atomic max
+// on one word: 106 -> 75 us at 128^3, 218 MB)
 template <int DIM>
-__global__ __launch_bounds__(kBlock) void k_visc_residual(ViscArgs A, Geo<DIM> g, Stat* st) {
+__global__ __launch_bounds__(kBlock) void k_visc_residual(ViscArgs A, Geo<DIM> g, Part* __restrict__ part) {
+  __shared__ double smax[kBlock / 64];
+  __shared__ unsigned long long snan[kBlock / 64];
   double m = 0.;
-  const idx_t n = g.ncell(), stride = (idx_t)gridDim.x * kBlock;
-  for (idx_t idx = logical_block() * kBlock + threadIdx.x; idx < n; idx += stride) {
+  unsigned long long nans = 0;
+  const idx_t idx = logical_block() * kBlock + threadIdx.x;
+  if (idx < g.ncell()) {
     int x[3];
     g.decode(idx, x);
     VAxes<DIM> X;
@@ -369,11 +516,24 @@ __global__ __launch_bounds__(kBlock) void k_visc_residual(ViscArgs A, Geo<DIM> g
       const double v =
           (A.r[c][idx] - visc_lambda<DIM>(A, mu, dtr, x, c) * u0) + dtr * visc_terms<DIM, true>(N, mu, c) / (A.D * A.D);
       A.out[c][idx] = v;
-      if (v != v) atomicAdd(&st->nans, 1ull);
+      if (v != v) nans++;
       else m = fmax(m, fabs(v));
     }
   }
-  block_max_to(st, m);
+  m = wave_max(m);
+  for (int o = 32; o > 0; o >>= 1) nans += __shfl_xor(nans, o, 64);
+  if ((threadIdx.x & 63) == 0) {
+    smax[threadIdx.x >> 6] = m;
+    snan[threadIdx.x >> 6] = nans;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < kBlock / 64; i++) {
+      m = fmax(m, smax[i]);
+      nans += snan[i];
+    }
+    part[blockIdx.x] = Part{m, nans};
+  }
 }
 
 }  // namespace bmg

@@ -240,3 +240,38 @@ def test_viscosity_explicit_bitexact(dim, depth, axi):
     assert sg["resb"] == so["resb"] and sg["i"] == 0
     for c in range(dim):
         assert np.array_equal(ug[c], uo[c]), c
+
+
+@pytest.mark.parametrize("dim,depth", [(2, 3), (2, 4), (2, 5), (3, 3), (3, 6)])
+def test_viscosity_coarse_workgroup_bitexact(dim, depth):
+    """Grids below, at and above the size whose levels all run in one
+    workgroup, periodic along x, with large coefficient jumps."""
+    print("case viscosity coarse", dim, depth, flush=True)
+    u, mu, rho = _problem(dim, depth, 31 * dim + depth, True)
+    for c in range(dim):  # face n is face 0 along a periodic dimension
+        if c == 0:
+            mu[c][-1] = mu[c][0]
+    g = bmg.Grid(dim, depth)
+    g.set_periodic(0)
+    g.set_tolerance(1e-7)
+    o = Viscosity(dim, depth)
+    o.smoother = "rbgs"
+    o.TOLERANCE = 1e-7
+    o.periodic = tuple([True] + [False] * (dim - 1))
+    o.set_coefficients(mu, rho)
+    uo, so, _ = o.solve(u, 0.003)
+    ug = [x.copy() for x in u]
+    sg = g.viscosity(ug, mu=mu, rho=rho, dt=0.003)
+    assert (sg["i"], sg["resb"], sg["resa"]) == (so["i"], so["resb"], so["resa"])
+    for c in range(dim):
+        assert np.array_equal(ug[c], uo[c]), c
+
+
+def test_viscosity_counts_nan():
+    print("case viscosity nan", flush=True)
+    u, mu, rho = _problem(3, 4, 5, False)
+    u[1][3, 4, 5] = np.nan
+    g = bmg.Grid(3, 4)
+    g.set_niter(2)
+    with pytest.raises(bmg.BMGError):
+        g.viscosity(u, mu=mu, rho=rho, dt=0.01)
