@@ -106,6 +106,12 @@ struct bmg_grid {
   Stat* stat = nullptr;
   double* partial = nullptr;
   double* scalar = nullptr;
+  // pinned host memory that the reductions' last kernels write (null: they
+  // write stat and scalar, copied back after each)
+  struct HostStat {
+    Stat stat;
+    double sum;
+  }* host = nullptr;
   int npartial = 1024;
   bool allocated_precision[2] = {false, false};
   // profiling
@@ -265,6 +271,33 @@ void prof_collect(bmg_grid* g) {
 int check_launch() {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(BMG_ERR_HIP, "kernel launch failed: %s", hipGetErrorString(e));
+  return BMG_OK;
+}
+
+// where the reductions' last kernels write, and the results on the host once
+// the stream has got there.  A copy of 16 bytes to pageable memory costs the
+// host about 15 us on top of the wait, in every cycle.
+Stat* stat_out(bmg_grid* g) { return g->host ? &g->host->stat : g->stat; }
+double* sum_out(bmg_grid* g) { return g->host ? &g->host->sum : g->scalar; }
+
+int read_stat(bmg_grid* g, double* maxres, unsigned long long* nans) {
+  Stat st;
+  if (!g->host) HIPCHECK(hipMemcpyAsync(&st, g->stat, sizeof st, hipMemcpyDeviceToHost, g->stream));
+  HIPCHECK(hipStreamSynchronize(g->stream));
+  if (g->host) {
+    const volatile Stat* h = &g->host->stat;
+    st.maxbits = h->maxbits;
+    st.nans = h->nans;
+  }
+  memcpy(maxres, &st.maxbits, sizeof *maxres);
+  if (nans) *nans += st.nans;
+  return BMG_OK;
+}
+
+int read_sum(bmg_grid* g, double* sum) {
+  if (!g->host) HIPCHECK(hipMemcpyAsync(sum, g->scalar, sizeof(double), hipMemcpyDeviceToHost, g->stream));
+  HIPCHECK(hipStreamSynchronize(g->stream));
+  if (g->host) *sum = *(const volatile double*)&g->host->sum;
   return BMG_OK;
 }
 
@@ -1165,14 +1198,16 @@ int mg_cycle_t(bmg_grid* g, int nrelax, int minlevel, int maxlevel, bool defer) 
         }
       }
       // one thread per coarse cell on the large 2D/3D levels
-      if (done) {
-      } else if (DIM >= 2 && lv.ncell >= (1u << 15)) {
-        hipLaunchKernelGGL((k_prolong_children<DIM, T>), dim3(nblocks(g->L[l - 1].ncell)), dim3(kBlock), 0,
-                           g->stream, (const T*)g->L[l - 1].da[0], (T*)lv.da[dst], gf, bcc);
-      } else {
+      if constexpr (DIM >= 2) {
+        if (!done && lv.ncell >= (1u << 15)) {
+          hipLaunchKernelGGL((k_prolong_children<DIM, T>), dim3(nblocks(g->L[l - 1].ncell)), dim3(kBlock), 0,
+                             g->stream, (const T*)g->L[l - 1].da[0], (T*)lv.da[dst], gf, bcc);
+          done = true;
+        }
+      }
+      if (!done)
         hipLaunchKernelGGL((k_prolong<DIM, T>), dim3(nblocks(lv.ncell)), dim3(kBlock), 0, g->stream,
                            (const T*)g->L[l - 1].da[0], (T*)lv.da[dst], gf, bcc);
-      }
     }
     TRY(check_launch());
     int cur = dst, rc = BMG_OK;
@@ -1289,7 +1324,7 @@ int residual_t(bmg_grid* g, double* maxres, bool force64, unsigned long long* na
           const double* da = corr ? (const double*)lf.da[0] : nullptr;
           corr_residual3<double, double>(g, af, lamf, nb, da, g->res64, nullptr, (double*)coarse, k, g3, bc, D, nch);
         }
-        hipLaunchKernelGGL(k_reduce_stat, dim3(1), dim3(1024), 0, g->stream, g->part, (int)nb, g->stat);
+        hipLaunchKernelGGL(k_reduce_stat, dim3(1), dim3(1024), 0, g->stream, g->part, (int)nb, stat_out(g));
       }
       TRY(check_launch());
       if (corr) {
@@ -1297,14 +1332,7 @@ int residual_t(bmg_grid* g, double* maxres, bool force64, unsigned long long* na
         g->pending_correct = false;
       }
       if (!force64) g->coarse_res_fresh = true;
-      Stat st;
-      HIPCHECK(hipMemcpyAsync(&st, g->stat, sizeof st, hipMemcpyDeviceToHost, g->stream));
-      HIPCHECK(hipStreamSynchronize(g->stream));
-      double m;
-      memcpy(&m, &st.maxbits, sizeof m);
-      *maxres = m;
-      if (nans) *nans += st.nans;
-      return BMG_OK;
+      return read_stat(g, maxres, nans);
     }
   }
   // bricks of whole 2^DIM child groups: the fused residual + restriction
@@ -1321,38 +1349,31 @@ int residual_t(bmg_grid* g, double* maxres, bool force64, unsigned long long* na
     else
       hipLaunchKernelGGL((k_residual_restrict<DIM, double>), dim3(nb), dim3(kBlock), 0, g->stream, g->a, g->b,
                          g->res64, (double*)coarse, (double*)nullptr, k, geo, bc, D, g->part);
-    hipLaunchKernelGGL(k_reduce_stat, dim3(1), dim3(1024), 0, g->stream, g->part, (int)nb, g->stat);
+    hipLaunchKernelGGL(k_reduce_stat, dim3(1), dim3(1024), 0, g->stream, g->part, (int)nb, stat_out(g));
     if (!force64) g->coarse_res_fresh = true;
   } else {
-    hipLaunchKernelGGL(k_stat_reset, dim3(1), dim3(64), 0, g->stream, g->stat);
     ProfScope ps(g, PROF_RESIDUAL);
+    // (g->part holds a partial per kBlock cells)
+    const unsigned nb = nblocks(lf.ncell);
     if (mixed)
-      hipLaunchKernelGGL((k_residual<DIM, float>), dim3(nblocks(lf.ncell)), dim3(kBlock), 0, g->stream, g->a,
-                         g->b, (float*)lf.res, keep64 ? g->res64 : (double*)nullptr, k, geo, bc, D, g->stat);
+      hipLaunchKernelGGL((k_residual<DIM, float>), dim3(nb), dim3(kBlock), 0, g->stream, g->a, g->b, (float*)lf.res,
+                         keep64 ? g->res64 : (double*)nullptr, k, geo, bc, D, g->part);
     else
-      hipLaunchKernelGGL((k_residual<DIM, double>), dim3(nblocks(lf.ncell)), dim3(kBlock), 0, g->stream, g->a,
-                         g->b, g->res64, (double*)nullptr, k, geo, bc, D, g->stat);
+      hipLaunchKernelGGL((k_residual<DIM, double>), dim3(nb), dim3(kBlock), 0, g->stream, g->a, g->b, g->res64,
+                         (double*)nullptr, k, geo, bc, D, g->part);
+    hipLaunchKernelGGL(k_reduce_stat, dim3(1), dim3(1024), 0, g->stream, g->part, (int)nb, stat_out(g));
   }
   TRY(check_launch());
-  Stat st;
-  HIPCHECK(hipMemcpyAsync(&st, g->stat, sizeof st, hipMemcpyDeviceToHost, g->stream));
-  HIPCHECK(hipStreamSynchronize(g->stream));
-  double m;
-  memcpy(&m, &st.maxbits, sizeof m);
-  *maxres = m;
-  if (nans) *nans += st.nans;
-  return BMG_OK;
+  return read_stat(g, maxres, nans);
 }
 
-int sum_b(bmg_grid* g, double* out) {
+// the sum of b; read_sum() fetches it (no wait here)
+int sum_b(bmg_grid* g) {
   Level& lf = g->L[g->depth];
   int np = (int)std::min<size_t>((size_t)g->npartial, nblocks(lf.ncell));
   hipLaunchKernelGGL(k_sum_partial, dim3(np), dim3(kBlock), 0, g->stream, g->b, lf.ncell, g->partial);
-  hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(64), 0, g->stream, g->partial, np, g->scalar);
-  TRY(check_launch());
-  HIPCHECK(hipMemcpyAsync(out, g->scalar, sizeof(double), hipMemcpyDeviceToHost, g->stream));
-  HIPCHECK(hipStreamSynchronize(g->stream));
-  return BMG_OK;
+  hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(kBlock), 0, g->stream, g->partial, np, sum_out(g));
+  return check_launch();
 }
 
 // restriction ({alpha, lambda}), poisson.h:418-420 in FP64, then the FP32
@@ -1565,10 +1586,11 @@ int mg_solve_impl(bmg_grid* g, double tolerance, int nrelax, int minlevel, bmg_m
   bmg_mgstats s;
   memset(&s, 0, sizeof s);
   unsigned long long nans = 0;
-  TRY(sum_b(g, &s.sum));
+  TRY(sum_b(g));
   s.nrelax = nrelax > 0 ? nrelax : 4;
   double resb;
   TRY(dispatch_residual(g, &s.resb, false, &nans));
+  TRY(read_sum(g, &s.sum));
   resb = s.resa = s.resb;
   if (tolerance == 0.) tolerance = g->TOLERANCE;
   for (s.i = 0; s.i < g->NITERMAX && (s.i < g->NITERMIN || s.resa > tolerance); s.i++) {
@@ -1743,6 +1765,12 @@ int grid_create(bmg_grid** out, int dimension, int depth, double L0, double X0, 
   if (r == BMG_OK) r = dalloc((void**)&g->partial, g->npartial * sizeof(double));
   if (r == BMG_OK) r = dalloc((void**)&g->part, (nf / kBlock + 1) * sizeof(Part));
   if (r == BMG_OK) r = dalloc((void**)&g->scalar, sizeof(double));
+  // (bmg_poisson_noalloc allocates nothing)
+  if (r == BMG_OK && !t_arena &&
+      hipHostMalloc((void**)&g->host, sizeof *g->host, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
+    g->host = nullptr;
+    (void)hipGetLastError();
+  }
   if (r == BMG_OK) r = alloc_levels(g);
   if (r == BMG_OK) {
     // every field starts at zero (reset (all, 0.), grid/multigrid.h:758)
@@ -1803,6 +1831,7 @@ int bmg_grid_free(bmg_grid* g) {
   dfreet(g->res64);
   for (int b = 0; b < 6; b++) dfreet(g->bc_c[b]);
   dfreet(g->stat);
+  if (g->host) (void)hipHostFree(g->host);
   dfreet(g->partial);
   dfreet(g->part);
   dfreet(g->scalar);
@@ -2801,14 +2830,9 @@ struct Visc {
     const unsigned nb = nblocks(lf.ncell);
     hipLaunchKernelGGL((k_visc_residual<DIM>), dim3(nb), dim3(kBlock), 0, g->stream,
                        args(g->depth, u, lv(g->depth, VS_RES), g->visc_r), geo, g->part);
-    hipLaunchKernelGGL(k_reduce_stat, dim3(1), dim3(1024), 0, g->stream, g->part, (int)nb, g->stat);
+    hipLaunchKernelGGL(k_reduce_stat, dim3(1), dim3(1024), 0, g->stream, g->part, (int)nb, stat_out(g));
     TRY(check_launch());
-    Stat st;
-    HIPCHECK(hipMemcpyAsync(&st, g->stat, sizeof st, hipMemcpyDeviceToHost, g->stream));
-    HIPCHECK(hipStreamSynchronize(g->stream));
-    memcpy(maxres, &st.maxbits, sizeof(double));
-    *nans += st.nans;
-    return BMG_OK;
+    return read_stat(g, maxres, nans);
   }
 
   // viscosity_explicit (viscosity.h:180-190): resb = residual_viscosity
@@ -2909,11 +2933,10 @@ struct Visc {
       HIPCHECK(hipMemcpyAsync(g->visc_r[c], u[c], lf.ncell * sizeof(double), hipMemcpyDeviceToDevice, g->stream));
       int np = (int)std::min<size_t>((size_t)g->npartial, nblocks(lf.ncell));
       hipLaunchKernelGGL(k_sum_partial, dim3(np), dim3(kBlock), 0, g->stream, g->visc_r[c], lf.ncell, g->partial);
-      hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(64), 0, g->stream, g->partial, np, g->scalar);
+      hipLaunchKernelGGL(k_sum_final, dim3(1), dim3(kBlock), 0, g->stream, g->partial, np, sum_out(g));
       TRY(check_launch());
       double sc = 0.;
-      HIPCHECK(hipMemcpyAsync(&sc, g->scalar, sizeof(double), hipMemcpyDeviceToHost, g->stream));
-      HIPCHECK(hipStreamSynchronize(g->stream));
+      TRY(read_sum(g, &sc));
       s.sum += sc;
     }
     restrict_coefficients();

@@ -575,37 +575,6 @@ __global__ __launch_bounds__(kBlock) void k_prolong(const T* __restrict__ coarse
   fine[idx] = bilinear_at<DIM, T>(coarse, gc, bcc, c);
 }
 
-// the same prolongation, one thread per coarse cell: its 2^DIM children
-// (bilinear_at each, sharing the coarse loads), the two children along the
-// last dimension written as one vector
-template <int DIM, typename T>
-__global__ __launch_bounds__(kBlock) void k_prolong_children(const T* __restrict__ coarse, T* __restrict__ fine,
-                                                             Geo<DIM> gf, BCH bcc) {
-  using V2 = typename Vec2<T>::type;
-  Geo<DIM> gc{gf.n >> 1, gf.log2n - 1};
-  idx_t idx = logical_block() * kBlock + threadIdx.x;
-  if (idx >= gc.ncell()) return;
-  int cc[3];
-  gc.decode(idx, cc);
-  const int nb = DIM == 3 ? 4 : 2;  // children groups along the other dimensions
-#pragma unroll
-  for (int m = 0; m < nb; m++) {
-    int c[3] = {2 * cc[0], 2 * cc[1], 2 * cc[2]};
-    if (DIM == 3) {
-      c[0] += m >> 1;
-      c[1] += m & 1;
-    } else {
-      c[0] += m;
-    }
-    V2 v;
-    v.x = bilinear_at<DIM, T>(coarse, gc, bcc, c);
-    c[DIM - 1] += 1;
-    v.y = bilinear_at<DIM, T>(coarse, gc, bcc, c);
-    c[DIM - 1] -= 1;
-    *reinterpret_cast<V2*>(fine + gf.index(c)) = v;
-  }
-}
-
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_fill(T* __restrict__ f, size_t n, T v) {
   size_t idx = (size_t)blockIdx.x * kBlock + threadIdx.x;
@@ -795,23 +764,50 @@ __device__ __forceinline__ double residual_cell(const double* __restrict__ a, co
   return r;
 }
 
+// a block's max |res| and NaN count, folded by k_reduce_stat
+struct Part {
+  double max;
+  unsigned long long nans;
+};
+
+__device__ __forceinline__ void block_part(double m, unsigned long long nans, Part* out) {
+  __shared__ double smax[kBlock / 64];
+  __shared__ unsigned long long snan[kBlock / 64];
+  m = wave_max(m);
+  for (int o = 32; o > 0; o >>= 1) nans += __shfl_xor(nans, o, 64);
+  if ((threadIdx.x & 63) == 0) {
+    smax[threadIdx.x >> 6] = m;
+    snan[threadIdx.x >> 6] = nans;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < kBlock / 64; i++) {
+      m = fmax(m, smax[i]);
+      nans += snan[i];
+    }
+    *out = Part{m, nans};
+  }
+}
+
 // residual of `a` on the finest level, writes res in the cycle precision TO
 template <int DIM, typename TO>
 __global__ __launch_bounds__(kBlock) void k_residual(const double* __restrict__ a, const double* __restrict__ b,
                                                      TO* __restrict__ res, double* __restrict__ res64,
-                                                     Coef<double> k, Geo<DIM> g, BCA bc, double D, Stat* st) {
+                                                     Coef<double> k, Geo<DIM> g, BCA bc, double D,
+                                                     Part* __restrict__ part) {
   idx_t idx = logical_block() * kBlock + threadIdx.x;
   double m = 0.;
+  unsigned long long nans = 0;
   if (idx < g.ncell()) {
     int c[3];
     g.decode(idx, c);
     double r = residual_cell<DIM>(a, b, k, g, bc, idx, c, D);
     res[idx] = (TO)r;
     if (res64) res64[idx] = r;
-    if (r != r) atomicAdd(&st->nans, 1ull);
+    if (r != r) nans = 1;
     else m = fabs(r);
   }
-  block_max_to(st, m);
+  block_part(m, nans, part + blockIdx.x);
 }
 
 // deterministic two-stage sum (sum of b, poisson.h:163-167)
@@ -830,10 +826,17 @@ __global__ __launch_bounds__(kBlock) void k_sum_partial(const double* __restrict
   }
 }
 
-__global__ void k_sum_final(const double* __restrict__ part, int np, double* __restrict__ out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
+// (the partials, at most kSumParts, come from LDS: one thread reading them
+// from memory one by one took 66 us for 1024)
+constexpr int kSumParts = 1024;
+__global__ __launch_bounds__(kBlock) void k_sum_final(const double* __restrict__ part, int np,
+                                                      double* __restrict__ out) {
+  __shared__ double sh[kSumParts];
+  for (int i = threadIdx.x; i < np; i += kBlock) sh[i] = part[i];
+  __syncthreads();
+  if (threadIdx.x == 0) {
     double s = 0.;
-    for (int i = 0; i < np; i++) s += part[i];
+    for (int i = 0; i < np; i++) s += sh[i];
     *out = s;
   }
 }
@@ -1200,11 +1203,6 @@ __global__ __launch_bounds__(kBlock) void k_wall_from_first(const double* __rest
 // and writes the 32 (3D) or 64 (2D) coarse residuals that restriction_average
 // makes of them, summed in foreach_child order.  The per-block max |res| and
 // NaN count go to `part`; k_reduce_stat folds them (no contended atomics).
-
-struct Part {
-  double max;
-  unsigned long long nans;
-};
 
 template <int DIM, typename TO>
 __global__ __launch_bounds__(kBlock) void k_residual_restrict(const double* __restrict__ a, const double* __restrict__ b,

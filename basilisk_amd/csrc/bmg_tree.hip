@@ -787,6 +787,12 @@ struct bmg_tree {
   // only bmg_tree_relax reads what it would have written
   int da_level = -1;
   TStat* stat = nullptr;
+  // pinned host memory that the reductions' last kernels write (null: copied
+  // back from stat and scalar); allocated with the stream
+  struct HostStat {
+    TStat stat;
+    double sum;
+  }* host = nullptr;
   double *part = nullptr, *scalar = nullptr;
   hipStream_t own_stream = nullptr, stream = nullptr;
   // field values kept across a recompilation, in leaf order
@@ -1755,6 +1761,10 @@ int ensure(bmg_tree* t) {
       return bmg::fail(BMG_ERR_HIP, "no HIP device available");
     HIPCHECK(hipStreamCreateWithFlags(&t->own_stream, hipStreamDefault));
     t->stream = t->own_stream;
+    if (hipHostMalloc((void**)&t->host, sizeof *t->host, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
+      t->host = nullptr;
+      (void)hipGetLastError();
+    }
   }
   if (t->topo.dirty || !t->compiled) return compile(t);
   return BMG_OK;
@@ -2128,6 +2138,7 @@ void residual_kernels(bmg_tree* t) {
   const double* lam = t->lambda_field ? t->lam64 : nullptr;
   k_t_leaf_res<DIM, T><<<(unsigned)S.first_block[S.n], kB, 0, t->stream>>>(
       S, t->a, t->b, t->g[0], t->g[1], t->g[2], x.nbr, lam, t->lambda_c, t->res64, F<T>(t->res), t->stat);
+  if (t->host) k_t_stat_out<<<1, 64, 0, t->stream>>>(t->stat, &t->host->stat);
 }
 
 // runs `launches` (kernel launches on t->stream only) as a captured graph,
@@ -2162,9 +2173,14 @@ int residual(bmg_tree* t, double* maxres) {
     return BMG_OK;
   }));
   TStat st;
-  HIPCHECK(hipMemcpyAsync(&st, t->stat, sizeof st, hipMemcpyDeviceToHost, t->stream));
+  if (!t->host) HIPCHECK(hipMemcpyAsync(&st, t->stat, sizeof st, hipMemcpyDeviceToHost, t->stream));
   HIPCHECK(hipStreamSynchronize(t->stream));
   HIPCHECK(hipGetLastError());
+  if (t->host) {
+    const volatile TStat* h = &t->host->stat;
+    st.maxbits = h->maxbits;
+    st.nans = h->nans;
+  }
   double m;
   memcpy(&m, &st.maxbits, sizeof m);
   *maxres = m;
@@ -2308,9 +2324,10 @@ int sum_b(bmg_tree* t, double* out) {
   const DevIndex& x = t->ix;
   int np = (int)std::min<long>(1024, std::max<long>(1, (long)nb_(x.nleaf)));
   k_t_sum_partial<<<np, kB, 0, t->stream>>>(x.leaf_gs, x.nleaf, t->b, t->part);
-  k_t_sum_final<<<1, 64, 0, t->stream>>>(t->part, np, t->scalar);
-  HIPCHECK(hipMemcpyAsync(out, t->scalar, sizeof(double), hipMemcpyDeviceToHost, t->stream));
+  k_t_sum_final<<<1, kB, 0, t->stream>>>(t->part, np, t->host ? &t->host->sum : t->scalar);
+  if (!t->host) HIPCHECK(hipMemcpyAsync(out, t->scalar, sizeof(double), hipMemcpyDeviceToHost, t->stream));
   HIPCHECK(hipStreamSynchronize(t->stream));
+  if (t->host) *out = *(const volatile double*)&t->host->sum;
   return BMG_OK;
 }
 
@@ -2637,6 +2654,7 @@ int bmg_tree_free(bmg_tree* t) {
     (void)hipEventDestroy(u.second.second);
   }
   for (hipEvent_t e : t->ev_pool) (void)hipEventDestroy(e);
+  if (t->host) (void)hipHostFree(t->host);
   if (t->own_stream) (void)hipStreamDestroy(t->own_stream);
   (void)hipGetLastError();
   delete t;

@@ -598,12 +598,22 @@ __global__ __launch_bounds__(kB) void k_t_sum_partial(const int* __restrict__ le
   }
 }
 
-__global__ void k_t_sum_final(const double* __restrict__ part, int np, double* __restrict__ out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
+// (the partials, at most kSumParts, come from LDS, see k_sum_final)
+constexpr int kSumParts = 1024;
+__global__ __launch_bounds__(kB) void k_t_sum_final(const double* __restrict__ part, int np, double* __restrict__ out) {
+  __shared__ double sh[kSumParts];
+  for (int i = threadIdx.x; i < np; i += kB) sh[i] = part[i];
+  __syncthreads();
+  if (threadIdx.x == 0) {
     double s = 0.;
-    for (int i = 0; i < np; i++) s += part[i];
+    for (int i = 0; i < np; i++) s += sh[i];
     *out = s;
   }
+}
+
+// the residual's statistics to pinned host memory
+__global__ void k_t_stat_out(const TStat* __restrict__ st, TStat* __restrict__ out) {
+  if (threadIdx.x == 0) *out = *st;
 }
 
 // --- small operations batched into one workgroup --------------------------

@@ -495,8 +495,6 @@ __global__ __launch_bounds__(kViscThreads<DIM>) void k_visc_coarse(ViscCoarse A)
 // on one word: 106 -> 75 us at 128^3, 218 MB)
 template <int DIM>
 __global__ __launch_bounds__(kBlock) void k_visc_residual(ViscArgs A, Geo<DIM> g, Part* __restrict__ part) {
-  __shared__ double smax[kBlock / 64];
-  __shared__ unsigned long long snan[kBlock / 64];
   double m = 0.;
   unsigned long long nans = 0;
   const idx_t idx = logical_block() * kBlock + threadIdx.x;
@@ -520,20 +518,7 @@ __global__ __launch_bounds__(kBlock) void k_visc_residual(ViscArgs A, Geo<DIM> g
       else m = fmax(m, fabs(v));
     }
   }
-  m = wave_max(m);
-  for (int o = 32; o > 0; o >>= 1) nans += __shfl_xor(nans, o, 64);
-  if ((threadIdx.x & 63) == 0) {
-    smax[threadIdx.x >> 6] = m;
-    snan[threadIdx.x >> 6] = nans;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int i = 1; i < kBlock / 64; i++) {
-      m = fmax(m, smax[i]);
-      nans += snan[i];
-    }
-    part[blockIdx.x] = Part{m, nans};
-  }
+  block_part(m, nans, part + blockIdx.x);
 }
 
 }  // namespace bmg
