@@ -707,8 +707,11 @@ struct DevIndex {
   int* halo_end_d = nullptr;
   int nstage = 0;
   std::vector<int> halo_end;  // [stage * (depth + 1) + level]: end of the stage's cells up to that level
-  int* crec = nullptr;        // per level: the first child record (of the next level) of every nonleaf record
-  std::vector<int> crec_off;
+  // restriction in one launch: its base level (-1: none has enough records)
+  // and per level from there on the first descendant of every base record
+  int rbase = -1;
+  int* drec = nullptr;
+  std::vector<int> drec_off;
   BoxRule* box = nullptr;
   FaceOp* fops = nullptr;
   FaceAvg *hf = nullptr, *fr = nullptr;
@@ -881,7 +884,7 @@ void free_device(bmg_tree* t) {
   drop_graphs(t);
   DevIndex& x = t->ix;
   for (void* p : {(void*)x.nbr, (void*)x.rec_self, (void*)x.rec_child0, (void*)x.rec_ring, (void*)x.colour,
-                  (void*)x.leaf_gs, (void*)x.lvl_leaves, (void*)x.col_list, (void*)x.col_nbr, (void*)x.halo, (void*)x.halo_end_d, (void*)x.crec, (void*)x.box, (void*)x.fops, (void*)x.hf, (void*)x.fr,
+                  (void*)x.leaf_gs, (void*)x.lvl_leaves, (void*)x.col_list, (void*)x.col_nbr, (void*)x.halo, (void*)x.halo_end_d, (void*)x.drec, (void*)x.box, (void*)x.fops, (void*)x.hf, (void*)x.fr,
                   (void*)x.fp, (void*)x.fc, (void*)x.fv_gs, (void*)x.fv_d, (void*)x.fc_tmp, (void*)x.lvinfo})
     dfree_(p);
   x = DevIndex();
@@ -1417,21 +1420,27 @@ int compile(bmg_tree* t) {
     TRY(upload(&x.halo_end_d, x.halo_end));
   }
   // the children of nonleaf record k of a level are active cells nch k ..
-  // of the next one, so its child records are a run
-  x.crec_off.assign(D + 1, 0);
-  {
-    std::vector<int> crec;
-    for (int l = 0; l < D; l++) {
-      x.crec_off[l] = (int)crec.size();
-      size_t q = 0;
-      for (int k = 0; k <= x.n_nonleaf[l]; k++) {
-        if (k < x.n_nonleaf[l] && rchild[(size_t)x.rec_off[l] + k] != x.off[l + 1] + k * nch) ok = false;
-        while (q < nonleaf[l + 1].size() && nonleaf[l + 1][q] < k * nch) q++;
-        crec.push_back((int)q);
+  // of the next one, so its child records are a run, and so on down
+  x.drec_off.assign(D + 1, 0);
+  x.rbase = x.lneed;
+  while (x.rbase < D && x.n_nonleaf[x.rbase] < kRestrictBase) x.rbase++;
+  if (x.rbase == D) x.rbase = -1;
+  if (x.rbase >= 0) {
+    const int nbase = x.n_nonleaf[x.rbase];
+    std::vector<int> drec(nbase + 1);
+    for (int r = 0; r <= nbase; r++) drec[r] = r;
+    for (int l = x.rbase; l + 1 < D; l++) {
+      const std::vector<int>& down = nonleaf[l + 1];
+      for (int k = 0; k < x.n_nonleaf[l]; k++)
+        if (rchild[(size_t)x.rec_off[l] + k] != x.off[l + 1] + k * nch) ok = false;
+      x.drec_off[l + 1] = (int)drec.size();
+      for (int r = 0; r <= nbase; r++) {
+        const int k = drec[(size_t)x.drec_off[l] + r];
+        drec.push_back((int)(std::lower_bound(down.begin(), down.end(), k * nch) - down.begin()));
       }
     }
     if (!ok) return bmg::fail(BMG_ERR_ARG, "tree: children out of cache order");
-    TRY(upload(&x.crec, crec));
+    TRY(upload(&x.drec, drec));
   }
   clk.mark("compile: tables: halo cells");
   // fine-face averages: halo_face (all levels in one launch) and the face
@@ -1810,6 +1819,7 @@ Segs level_or_leaf_colour(const bmg_tree* t, int l, int c) {
   memset(&S, 0, sizeof S);
   int blocks = 0;
   for (int m = l; m >= 0; m--) {
+    if (m < l && !x.lcol_n[2 * m + c]) continue;  // (a block looks through the segments before its own)
     int s = S.n++;
     S.first_block[s] = blocks;
     S.abase[s] = x.abase[m];
@@ -1953,6 +1963,7 @@ struct Batcher {
     A.halo = x.halo;
     A.halo_end = x.halo_end_d;
     A.depth = x.depth;
+    A.lneed = x.lneed;
     A.box = x.box;
     A.fld[0] = f0;
     A.fld[1] = f1;
@@ -1997,28 +2008,26 @@ struct Batcher {
     k_t_prolong<T, DIM>
         <<<nb_(n), kB, 0, t->stream>>>(x.rec_ring + (size_t)r0 * NR, x.rec_child0 + r0, n, A.fld[f], x.box);
   }
-  // restriction of f to the levels m1 .. m0 (m1 >= m0): the levels from the
-  // first with kRestrictBase records on in one launch, a workgroup per run of
-  // records (one launch per level cost 2.3 us each on a chain of 6)
+  // restriction of f to the levels m1 .. m0 (m1 >= m0): those from the base
+  // level on in one launch, a workgroup per run of its records (one launch
+  // per level cost 2.3 us each on a chain of 6)
   void restrict_range(int f, int m1, int m0) {
-    int base = m0;
-    while (base < m1 && x.n_nonleaf[base] < kRestrictBase) base++;
-    if (m1 - base >= 1 && !small(x.n_nonleaf[m1])) {
+    const int lo = std::max(m0, x.rbase);
+    if (x.rbase >= 0 && m1 > lo && !small(x.n_nonleaf[m1])) {
       flush();
       RestrictLevels L;
       memset(&L, 0, sizeof L);
-      L.m0 = base;
+      L.m0 = lo;
       L.m1 = m1;
-      for (int m = base; m <= m1; m++) {
+      for (int m = lo; m <= m1; m++) {
         L.rec_off[m] = x.rec_off[m];
-        L.n[m] = x.n_nonleaf[m];
-        L.crec_off[m] = x.crec_off[m];
+        L.drec_off[m] = x.drec_off[m];
       }
-      const int n = x.n_nonleaf[base];
-      L.per_block = std::max(1, n / kRestrictBlocks);
-      k_t_restrict_tree<T, DIM><<<(unsigned)((n + L.per_block - 1) / L.per_block), kB, 0, t->stream>>>(
-          L, x.rec_self, x.rec_child0, x.crec, A.fld[f]);
-      m1 = base - 1;
+      L.nbase = x.n_nonleaf[x.rbase];
+      L.per_block = std::max(1, L.nbase / kRestrictBlocks);
+      k_t_restrict_tree<T, DIM><<<(unsigned)((L.nbase + L.per_block - 1) / L.per_block), kB, 0, t->stream>>>(
+          L, x.rec_self, x.rec_child0, x.drec, A.fld[f]);
+      m1 = lo - 1;
     }
     for (int m = m1; m >= m0; m--) restrict_level(f, m);
   }

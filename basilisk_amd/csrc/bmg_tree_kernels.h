@@ -164,36 +164,32 @@ __global__ __launch_bounds__(kB) void k_t_restrict(const int* __restrict__ self,
   t_restrict_one<T, DIM>(f, self[r], child0[r]);
 }
 
-// the levels m0 .. m1 of a restriction in one launch: a workgroup takes the
-// records [r0, r1) of level m0 and everything below them, the finest level
-// first, with a barrier between levels.  The records of a level are in cache
-// order, so the children of a run of records are the run that `crec` (the
-// first child record of every record, per level) bounds.
+// the levels m0 .. m1 of a restriction in one launch: a workgroup takes a run
+// of records of the base level (at or above m0 in the tree) and everything
+// below them, the finest level first, with a barrier between levels.  The
+// records of a level are in cache order, so the descendants of a run of
+// records are a run on every level, bounded by `drec` (per level, the first
+// descendant of every base record; walking down a table of children instead
+// cost a chain of loads, 6.6 instead of 5 us a launch).
 struct RestrictLevels {
-  int m0, m1, per_block;          // levels; records of level m0 per workgroup
-  int rec_off[kSeg], n[kSeg];     // records of each level
-  int crec_off[kSeg];             // its part of crec (n + 1 entries)
+  int m0, m1, nbase, per_block;              // levels; records of the base level, per workgroup
+  int rec_off[kSeg], drec_off[kSeg];         // records of each level, its part of drec (nbase + 1 entries)
 };
 
 template <typename T, int DIM>
 __global__ __launch_bounds__(kB) void k_t_restrict_tree(RestrictLevels L, const int* __restrict__ self,
-                                                        const int* __restrict__ child0, const int* __restrict__ crec,
+                                                        const int* __restrict__ child0, const int* __restrict__ drec,
                                                         T* f) {
   __shared__ int lo[kSeg], hi[kSeg];
-  if (threadIdx.x == 0) {
-    int a = min((int)blockIdx.x * L.per_block, L.n[L.m0]), b = min(a + L.per_block, L.n[L.m0]);
-    for (int m = L.m0;; m++) {
-      lo[m] = a;
-      hi[m] = b;
-      if (m == L.m1) break;
-      a = crec[L.crec_off[m] + a];
-      b = crec[L.crec_off[m] + b];
-    }
+  const int a = min((int)blockIdx.x * L.per_block, L.nbase), b = min(a + L.per_block, L.nbase);
+  const int q = L.m0 + (int)threadIdx.x;
+  if (q <= L.m1) {
+    lo[q] = L.rec_off[q] + drec[L.drec_off[q] + a];
+    hi[q] = L.rec_off[q] + drec[L.drec_off[q] + b];
   }
   __syncthreads();
   for (int m = L.m1; m >= L.m0; m--) {
-    for (int r = lo[m] + (int)threadIdx.x; r < hi[m]; r += kB)
-      t_restrict_one<T, DIM>(f, self[L.rec_off[m] + r], child0[L.rec_off[m] + r]);
+    for (int r = lo[m] + (int)threadIdx.x; r < hi[m]; r += kB) t_restrict_one<T, DIM>(f, self[r], child0[r]);
     __syncthreads();
   }
 }
@@ -664,7 +660,7 @@ struct TreeArgs {
   const TLevelInfo* lv;
   const int *rec_self, *rec_child0, *rec_ring, *lvl_leaves, *col_list, *col_nbr;
   const int *halo, *halo_end;  // halo cells by stage and level; per stage and level their end
-  int depth;
+  int depth, lneed;            // lneed: the coarsest level with leaves
   const BoxRule* box;
   T* fld[3];  // fields an operation can name (da, res, tmp; or `a` alone)
   const T* res;
@@ -674,11 +670,12 @@ struct TreeArgs {
 };
 
 template <typename T, int DIM>
-__device__ __forceinline__ void t_ops_cells(const TreeArgs<T>& A, const TOp& op) {
+__device__ __forceinline__ void t_ops_cells(const TreeArgs<T>& A, const TLevelInfo* lv, const TOp& op) {
   const int l = op.level;
   T* da = A.fld[0];
-  for (int m = l; m >= 0; m--) {
-    const TLevelInfo& L = A.lv[m];
+  // the level, then the leaves of the levels that have any
+  for (int m = l; m == l || m >= A.lneed; m--) {
+    const TLevelInfo& L = lv[m];
     if (op.code == TOP_RELAX) {
       const T Dm = (T)(A.L0 * (1. / (1 << m)));
       for (int c = op.arg < 0 ? 0 : op.arg; c <= (op.arg < 0 ? 1 : op.arg); c++) {
@@ -706,9 +703,15 @@ __device__ __forceinline__ void t_ops_cells(const TreeArgs<T>& A, const TOp& op)
 template <typename T, int DIM>
 __global__ __launch_bounds__(kOpsBlock) void k_t_ops(TOps P, TreeArgs<T> A) {
   constexpr int NR = DIM == 2 ? 9 : 27;
+  // the level table in LDS: an operation is a chain of dependent loads, and
+  // its extents are the first
+  __shared__ TLevelInfo lv[kSeg];
+  for (int i = threadIdx.x; i < (A.depth + 1) * (int)(sizeof(TLevelInfo) / 4); i += (int)blockDim.x)
+    ((int*)lv)[i] = ((const int*)A.lv)[i];
+  __syncthreads();
   for (int o = 0; o < P.n; o++) {
     const TOp op = P.op[o];
-    const TLevelInfo L = A.lv[op.level];
+    const TLevelInfo& L = lv[op.level];
     T* f = A.fld[op.field];
     switch (op.code) {
       case TOP_RESTRICT:
@@ -741,7 +744,7 @@ __global__ __launch_bounds__(kOpsBlock) void k_t_ops(TOps P, TreeArgs<T> A) {
         break;
       }
       default:
-        t_ops_cells<T, DIM>(A, op);
+        t_ops_cells<T, DIM>(A, lv, op);
     }
     __syncthreads();
   }
