@@ -682,7 +682,7 @@ __global__ __launch_bounds__(kBlock) void k_coef_grad(const double* __restrict__
   out[t] = v;
 }
 
-__global__ __launch_bounds__(kBlock) void k_lambda_grad(const double* __restrict__ a, const double* __restrict__ psi,
+[[maybe_unused]] static __global__ __launch_bounds__(kBlock) void k_lambda_grad(const double* __restrict__ a, const double* __restrict__ psi,
                                                         double* __restrict__ out, size_t n) {
   size_t t = (size_t)blockIdx.x * kBlock + threadIdx.x;
   if (t < n) out[t] = -psi[t] * a[t];
@@ -696,7 +696,7 @@ struct Stat {
   unsigned long long nans;     // number of NaN residuals
 };
 
-__global__ void k_stat_reset(Stat* s) {
+[[maybe_unused]] static __global__ void k_stat_reset(Stat* s) {
   if (threadIdx.x == 0) {
     s->maxbits = 0ull;
     s->nans = 0ull;
@@ -811,7 +811,7 @@ __global__ __launch_bounds__(kBlock) void k_residual(const double* __restrict__ 
 }
 
 // deterministic two-stage sum (sum of b, poisson.h:163-167)
-__global__ __launch_bounds__(kBlock) void k_sum_partial(const double* __restrict__ x, size_t n,
+[[maybe_unused]] static __global__ __launch_bounds__(kBlock) void k_sum_partial(const double* __restrict__ x, size_t n,
                                                         double* __restrict__ part) {
   __shared__ double sh[kBlock / 64];
   double v = 0.;
@@ -829,7 +829,7 @@ __global__ __launch_bounds__(kBlock) void k_sum_partial(const double* __restrict
 // (the partials, at most kSumParts, come from LDS: one thread reading them
 // from memory one by one took 66 us for 1024)
 constexpr int kSumParts = 1024;
-__global__ __launch_bounds__(kBlock) void k_sum_final(const double* __restrict__ part, int np,
+[[maybe_unused]] static __global__ __launch_bounds__(kBlock) void k_sum_final(const double* __restrict__ part, int np,
                                                       double* __restrict__ out) {
   __shared__ double sh[kSumParts];
   for (int i = threadIdx.x; i < np; i += kBlock) sh[i] = part[i];
@@ -1009,7 +1009,7 @@ __global__ __launch_bounds__(kBlock) void k_centered_gradient(CenteredArgs A, Ge
 }
 
 // correction (centered.h:322-327): u.x[] += dt*g.x[]
-__global__ __launch_bounds__(kBlock) void k_correction(double* __restrict__ u, const double* __restrict__ gx,
+[[maybe_unused]] static __global__ __launch_bounds__(kBlock) void k_correction(double* __restrict__ u, const double* __restrict__ gx,
                                                        double dt, size_t n) {
   const size_t idx = (size_t)blockIdx.x * kBlock + threadIdx.x;
   if (idx < n) u[idx] += dt * gx[idx];
@@ -1151,7 +1151,7 @@ struct ConvBatch {
   int nseg;
 };
 
-__global__ __launch_bounds__(kBlock) void k_convert_batch(ConvBatch B) {
+[[maybe_unused]] static __global__ __launch_bounds__(kBlock) void k_convert_batch(ConvBatch B) {
   const unsigned blk = blockIdx.x;
   // the segment of this block: the number of later segments starting at or
   // before it (independent loads of the increasing starts, not a chain)
@@ -1287,7 +1287,7 @@ __global__ __launch_bounds__(kBlock) void k_residual_restrict(const double* __re
   }
 }
 
-__global__ __launch_bounds__(1024) void k_reduce_stat(const Part* __restrict__ part, int np, Stat* st) {
+[[maybe_unused]] static __global__ __launch_bounds__(1024) void k_reduce_stat(const Part* __restrict__ part, int np, Stat* st) {
   __shared__ double smax[16];
   __shared__ unsigned long long snan[16];
   double m = 0.;

@@ -36,6 +36,7 @@
 
 #include "../../include/bmg.h"
 #include "bmg_internal.h"
+#include "bmg_tree_coarse.h"
 #include "bmg_tree_kernels.h"
 
 using namespace bmgt;
@@ -700,6 +701,7 @@ struct DevIndex {
   // the coarsest level with leaves or residual faces: the cycle and the
   // residual read no restricted value above it
   int lneed = 0;
+  int ctop = -1;  // the finest level that is a full grid in cache order, nothing coarser being a leaf (k_t_coarse)
   // the halo cells that relax, the initial guesses and the residual's faces
   // read, as 2^dim * record + child, by dependency stage (a cell interpolated
   // from halo cells of stage k - 1 has stage k) and then by level
@@ -1335,6 +1337,17 @@ int compile(bmg_tree* t) {
   x.lneed = D;
   for (int l = D; l >= 0; l--)
     if (x.leaf_n[l] || x.face_n[l] || x.n_prolong[l]) x.lneed = l;
+  x.ctop = 0;
+  for (int l = 1; l <= std::min({D, x.lneed, kCoarseTop}); l++) {
+    bool full = x.nA[l] == 1 << (dim * l);
+    for (int q = 0; full && q < x.nA[l]; q++) {
+      const IJK& a = T.active[l][q];
+      const int c[3] = {a.i - GH, a.j - GH, dim == 3 ? a.k - GH : 0};
+      full = (dim == 3 ? cache_index<3>(c, l) : cache_index<2>(c, l)) == q;
+    }
+    if (!full) break;
+    x.ctop = l;
+  }
   table<int> halo;
   {
     std::vector<size_t> hoff(D + 2, 0);
@@ -2031,6 +2044,38 @@ struct Batcher {
     }
     for (int m = m1; m >= m0; m--) restrict_level(f, m);
   }
+  // the levels minlevel .. coarse_top() of a red-black cycle in one launch
+  // (-1: none).  A thread per 2^dim block: 32^2, or 16^3, or 8^3 where a
+  // block's face values in FP64 leave no registers for more waves
+  int coarse_top(int minlevel, int maxlevel) const {
+    if (!t->batching || t->smoother != BMG_RELAX_RBGS || minlevel < 1) return -1;
+    const int cap = DIM == 2 ? 5 : t->alpha_field && sizeof(T) == 8 ? 3 : 4;
+    const int top = std::min({x.ctop, cap, maxlevel});
+    return top >= minlevel ? top : -1;
+  }
+  void coarse(int nrelax, int minlevel, int top) {
+    flush();
+    TreeCoarse<T> C;
+    memset((void*)&C, 0, sizeof C);
+    C.da = A.fld[0];
+    C.res = A.fld[1];
+    C.k = A.k;
+    C.nbr = x.nbr;
+    for (int b = 0; b < 6; b++) C.bc.sigma[b] = t->bc_kind[b] == BMG_BC_DIRICHLET ? -1 : 1;
+    C.bc.tree = 1;
+    C.minlevel = minlevel;
+    C.top = top;
+    C.nrelax = nrelax;
+    for (int l = minlevel; l <= top; l++) {
+      C.off[l] = x.off[l];
+      C.abase[l] = x.abase[l];
+      const T D = (T)delta(t, l);
+      C.D2[l] = D * D;
+    }
+    const unsigned nt = std::max(64u, 1u << (DIM * (top - 1)));
+    if (t->alpha_field) k_t_coarse<DIM, T, true><<<1, nt, 0, t->stream>>>(C);
+    else k_t_coarse<DIM, T, false><<<1, nt, 0, t->stream>>>(C);
+  }
   // what the cycle and the residual read of tree_boundary_level ({f}, l):
   // the restricted values down to the coarsest level with leaves and the
   // halo cells, a launch per dependency stage; ghosts are evaluated by
@@ -2263,8 +2308,11 @@ int cycle_kernels(bmg_tree* t, int nrelax, int minlevel, int maxlevel) {
   minlevel = std::min(minlevel, maxlevel);
   // restriction (res) of mg_cycle: relax reads res in the cells it relaxes,
   // so neither levels above minlevel nor halo cells nor ghosts
-  if (x.depth > minlevel) B.restrict_range(1, x.depth - 1, minlevel);
-  for (int l = minlevel; l <= maxlevel; l++) {
+  const int top = B.coarse_top(minlevel, maxlevel);
+  const int rlow = std::max(minlevel, top);
+  if (x.depth > rlow) B.restrict_range(1, x.depth - 1, rlow);
+  if (top >= 0) B.coarse(nrelax, minlevel, top);
+  for (int l = top >= 0 ? top + 1 : minlevel; l <= maxlevel; l++) {
     if (l == minlevel)
       B.fill(l);
     else
