@@ -1035,7 +1035,7 @@ int relax_level(bmg_grid* g, int l) {
 }
 
 template <int DIM, typename T>
-int coarse_block(bmg_grid* g, int nrelax, int minlevel, int top) {
+int coarse_block(bmg_grid* g, int nrelax, int minlevel, int top, bool* corrected) {
   static_assert(sizeof(CoarseArgs<T, DIM>) <= 4096, "kernel argument block too large");
   if (top >= kCoarseLevels || minlevel < 0 || minlevel > top)
     return fail(BMG_ERR_ARG, "internal: coarse levels %d..%d out of range", minlevel, top);
@@ -1061,6 +1061,10 @@ int coarse_block(bmg_grid* g, int nrelax, int minlevel, int top) {
   ProfScope ps(g, PROF_RELAX_COARSE);
   if constexpr (DIM >= 2) {
     if (coarse_in_lds(g)) {
+      if (top == g->depth) {
+        A.a = g->a;
+        *corrected = true;
+      }
       // a thread per block of the largest level
       const size_t blocks = g->L[top].ncell >> DIM;
       const dim3 nt((unsigned)std::max<size_t>(64, blocks));
@@ -1149,8 +1153,8 @@ int mg_cycle_t(bmg_grid* g, int nrelax, int minlevel, int maxlevel, bool defer) 
   }
   TRY(check_launch());
   // the coarse levels in one workgroup; they end in da[0]
-  if (use_block) TRY((coarse_block<DIM, T>(g, nrelax, minlevel, top)));
   bool corrected = false;
+  if (use_block) TRY((coarse_block<DIM, T>(g, nrelax, minlevel, top, &corrected)));
   for (int l = use_block ? top + 1 : minlevel; l <= maxlevel; l++) {
     Level& lv = g->L[l];
     // ping-pong sweeps start in da[flips & 1] so that they end in da[0]
@@ -1172,7 +1176,7 @@ int mg_cycle_t(bmg_grid* g, int nrelax, int minlevel, int maxlevel, bool defer) 
         TRY((tile_sweep<DIM, T>(g, l, ns, j == 0 && l > minlevel ? -1 : (nl - j) & 1, (nl - 1 - j) & 1,
                                 own && j == nl - 1)));
       }
-      corrected = own;
+      corrected |= own;
       continue;
     }
     const bool two = use_sweep2<DIM, T>(g, l);

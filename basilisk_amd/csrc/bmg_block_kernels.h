@@ -213,7 +213,8 @@ __global__ __launch_bounds__(kBlock) void k_prolong_children(const T* __restrict
 // Levels minlevel..top of the cycle (top of at most 16^3 or 32^2 cells):
 // restriction of res down to minlevel, then from minlevel up the zero
 // or bilinear initial guess and nrelax sweeps, a thread per block of the
-// level.  res and da of every level end in memory too.
+// level.  res and da of every level end in memory too.  On a grid that ends
+// there the correction is added as well (a launch of 4 us otherwise).
 //
 // NT: the blocks of the largest level it takes.  2D: 256 (32^2).  3D: 512
 // (16^3), but with a face field in FP64 a block's 60 values leave no
@@ -276,6 +277,7 @@ __global__ __launch_bounds__((kCoarseThreads<DIM, T, ALPHAF>)) void k_coarse_rb(
         }
         cur[0] = v;
         L.da[0] = v;
+        if (A.a && A.top == 0) A.a[0] += (double)v;
       }
       __syncthreads();
       continue;
@@ -340,6 +342,12 @@ __global__ __launch_bounds__((kCoarseThreads<DIM, T, ALPHAF>)) void k_coarse_rb(
         w.x = B.v[p];
         w.y = B.v[p + 1];
         *reinterpret_cast<typename Vec2<T>::type*>(L.da + at) = w;
+        if (A.a && l == A.top) {
+          double2 x = *reinterpret_cast<const double2*>(A.a + at);
+          x.x += (double)w.x;
+          x.y += (double)w.y;
+          *reinterpret_cast<double2*>(A.a + at) = x;
+        }
       }
     }
   }

@@ -2542,6 +2542,7 @@ template <typename T, int DIM>
 struct CoarseArgs {
   CoarseLevel<T, DIM> L[kCoarseLevels];
   int minlevel, top, nrelax, jacobi, gs;  // gs: the in-place Gauss-Seidel order, through da2
+  double* a;  // k_coarse_rb: where the finest level ends the cycle, the solution it corrects (or null)
 };
 
 template <int DIM, typename T>
