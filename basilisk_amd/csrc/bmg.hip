@@ -121,10 +121,12 @@ struct bmg_grid {
   int sweep2_min = 256;  // BMG_SWEEP2_MIN: smallest level edge of the two-sweep kernel (0: off)
   int grid_kind = BMG_GRID_MULTIGRID;  // ghost rule of edges and corners
   // the cycle as a HIP graph per (nrelax, minlevel, maxlevel, deferred
-  // correction, fresh coarse res); dropped whenever a kernel argument of the
-  // cycle could change (BMG_GRAPHS=0: plain launches)
+  // correction, fresh coarse res, the array it corrects); dropped whenever
+  // another kernel argument of the cycle could change (BMG_GRAPHS=0: plain
+  // launches).  The array: a and a2 swap with every deferred correction, so a
+  // cycle that corrects by itself has a graph for each of the two.
   bool use_graphs = true;
-  std::map<std::tuple<int, int, int, int, int>, hipGraphExec_t> cycle_graphs;
+  std::map<std::tuple<int, int, int, int, int, const double*>, hipGraphExec_t> cycle_graphs;
   std::vector<hipEvent_t> ev_pool;
   std::vector<std::pair<int, std::pair<hipEvent_t, hipEvent_t>>> ev_used;
   double prof_ms[PROF_N] = {0};
@@ -1472,8 +1474,10 @@ template <int DIM, typename T>
 int cycle_graph(bmg_grid* g, int nrelax, int minlevel, int maxlevel, bool defer) {
   // profiling records events around the kernels: plain launches then
   if (!g->use_graphs || g->prof) return mg_cycle_t<DIM, T>(g, nrelax, minlevel, maxlevel, defer);
+  const bool deferred = defer && maxlevel == g->depth;
   hipGraphExec_t& slot = g->cycle_graphs[std::make_tuple(nrelax, minlevel, maxlevel, (int)defer,
-                                                         (int)g->coarse_res_fresh)];
+                                                         (int)g->coarse_res_fresh,
+                                                         deferred ? (const double*)nullptr : (const double*)g->a)];
   if (!slot) {
     // capturing runs the host side of the cycle (its flags) but no kernel
     hipGraph_t graph = nullptr;
@@ -1493,7 +1497,7 @@ int cycle_graph(bmg_grid* g, int nrelax, int minlevel, int maxlevel, bool defer)
   } else {
     // the host side of mg_cycle_t
     g->coarse_res_fresh = false;
-    if (defer && maxlevel == g->depth) g->pending_correct = true;
+    if (deferred) g->pending_correct = true;
   }
   HIPCHECK(hipGraphLaunch(slot, g->stream));
   return BMG_OK;

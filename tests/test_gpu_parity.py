@@ -331,6 +331,36 @@ def test_cycle_graph_replays_equal_plain_launches(precision, depth, monkeypatch)
     assert np.array_equal(f0, f1)
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("box", ["walls", "periodic"])
+def test_cycle_graph_after_a_solve_corrects_the_current_solution(precision, box, monkeypatch):
+    """Every cycle of a solve on a 3D grid of 128^3 and more leaves its
+    correction to the residual, which writes a + da to a second array and
+    swaps the two.  A cycle that corrects by itself is captured with the
+    array of its time; after an odd number of swaps its replay would correct
+    the other one.  Cycles and one-cycle solves in turn, several replays with
+    either array, against plain launches."""
+    print("case graphs across solves", precision, box, flush=True)
+    kinds = [cases.BC_PERIODIC] * 6 if box == "periodic" else BC_MIXES["mixed"]
+    runs = []
+    for graphs in ("1", "0"):
+        monkeypatch.setenv("BMG_GRAPHS", graphs)
+        g = bmg.Grid(3, 7, smoother="rbgs", precision=precision)
+        cases.random_problem(g, 33, lam=-1.3, bcs=kinds)
+        g.restriction_alpha_lambda()
+        res = []
+        for it in range(5):
+            g.mg_cycle(2, 1)
+            res.append(g.residual())
+            g.set_niter(1 + it // 3, 1)
+            res.append(g.poisson(tolerance=1e-30, nrelax=2)["resa"])
+        g.mg_cycle(2, 1)
+        runs.append((res, g.get_a()))
+    (r0, a0), (r1, a1) = runs
+    assert r0 == r1
+    assert np.array_equal(a0, a1)
+
+
 def test_nan_is_reported():
     g = bmg.Grid(2, 5)
     b = np.zeros(g.shape())
