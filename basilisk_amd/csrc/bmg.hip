@@ -116,7 +116,7 @@ struct bmg_grid {
   bool allocated_precision[2] = {false, false};
   // profiling
   bool prof = false;
-  int rb_override = -1;  // BMG_RB_KERNEL: kernel for red-black levels of >= 4096 cells
+  int rb_override = -1;  // BMG_RB_KERNEL: kernel for red-black levels of >= 4096 cells (and none on chip)
   int rb_reverse = 1;    // black passes walk the blocks backwards (BMG_RB_REVERSE=0: forwards)
   int sweep2_min = 256;  // BMG_SWEEP2_MIN: smallest level edge of the two-sweep kernel (0: off)
   int grid_kind = BMG_GRID_MULTIGRID;  // ghost rule of edges and corners
@@ -776,21 +776,26 @@ int stream_chunk(int n) {
   return n >= 256 ? 16 : 8;
 }
 
-
+// whether the coarsest levels may run in k_coarse_rb: red-black in 2D and 3D,
+// unless a kernel from memory is asked for (BMG_RB_KERNEL, or the threads of
+// k_coarse_cycle by BMG_COARSE_BLOCK)
 bool coarse_in_lds(const bmg_grid* g) {
-  return g->smoother == BMG_RELAX_RBGS && g->dim >= 2 && g->rb_override < 0;
+  return g->smoother == BMG_RELAX_RBGS && g->dim >= 2 && g->rb_override < 0 && !size_knob("BMG_COARSE_BLOCK", 0);
 }
 
-// largest level that the single-workgroup coarse kernel takes (at most 4096
-// cells; BMG_COARSE_TOP overrides within that limit)
+// largest level that k_coarse_rb takes (kCoarseThreads blocks)
+int coarse_rb_top(const bmg_grid* g) {
+  return g->dim == 2 ? 5 : g->precision == BMG_FP64 && g->alpha_field ? 3 : 4;
+}
+
+// largest level of the single-workgroup coarse kernel (at most 4096 cells;
+// BMG_COARSE_TOP overrides within that limit: k_coarse_cycle takes what
+// k_coarse_rb has no threads for)
 int coarse_top(const bmg_grid* g) {
-  // levels of 512-1024 cells; red-black in 3D (k_coarse_rb, on chip) the
-  // 16^3 level too, unless its registers do not suffice: 12 us for its
+  // levels of 512-1024 cells; in 3D on chip the 16^3 level too: 12 us for its
   // sweeps in this kernel against two launches of 10 us by tiles and the
   // restriction's own (64^2: 8 us against 5 and 2)
-  const bool lds = coarse_in_lds(g), few = g->precision == BMG_FP64 && g->alpha_field;
-  int top = g->dim == 3 ? (lds && !few ? 4 : 3) : g->dim == 2 ? 5 : 10;
-  if (lds) return std::min(top, g->depth);
+  int top = coarse_in_lds(g) ? coarse_rb_top(g) : g->dim == 3 ? 3 : g->dim == 2 ? 5 : 10;
   if (const char* e = getenv("BMG_COARSE_TOP")) {
     int v = atoi(e), lim = g->dim == 3 ? 4 : g->dim == 2 ? 6 : 12;
     if (v >= 0 && v <= lim) top = v;
@@ -1062,7 +1067,7 @@ int coarse_block(bmg_grid* g, int nrelax, int minlevel, int top, bool* corrected
   A.gs = g->smoother == BMG_RELAX_GS;
   ProfScope ps(g, PROF_RELAX_COARSE);
   if constexpr (DIM >= 2) {
-    if (coarse_in_lds(g)) {
+    if (coarse_in_lds(g) && top <= coarse_rb_top(g)) {
       if (top == g->depth) {
         A.a = g->a;
         *corrected = true;
@@ -1075,7 +1080,7 @@ int coarse_block(bmg_grid* g, int nrelax, int minlevel, int top, bool* corrected
       return check_launch();
     }
   }
-  // threads of the workgroup (BMG_COARSE_BLOCK: a multiple of 64 up to 1024)
+  // threads of k_coarse_cycle (BMG_COARSE_BLOCK: a multiple of 64 up to 1024)
   size_t nt = size_knob("BMG_COARSE_BLOCK", 1024);
   if (nt > 1024 || nt % 64) nt = 1024;
   hipLaunchKernelGGL((k_coarse_cycle<DIM, T>), dim3(1), dim3((unsigned)nt), 0, g->stream, A);

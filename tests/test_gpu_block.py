@@ -107,3 +107,56 @@ def test_graph_replays_of_a_correcting_cycle():
             g.mg_cycle(3, 1)
             g.synchronize()
     assert np.array_equal(grids[0].get_a(), grids[1].get_a())
+
+
+def _coarse_launches(dim, depth, top, nrelax):
+    """launches of the coarse levels of a cycle: one workgroup for the levels
+    up to top, then per level a launch for every sweep (4^dim and 8^dim cells)
+    or for up to 4 (2D) or 2 (3D) sweeps"""
+    n = 1
+    for l in range(top + 1, depth):
+        n += nrelax if l < 4 else -(-nrelax // (4 if dim == 2 else 2))
+    return n
+
+
+@pytest.mark.parametrize("dim,depth,coef,precision,default,top",
+                         [(2, 7, "alpha", "fp64", 5, t) for t in (0, 2, 6)] + [(2, 7, "lam", "mixed", 5, 4)]
+                         + [(3, 5, "alpha", "fp64", 3, t) for t in (1, 4)]
+                         + [(3, 5, "", "fp64", 4, 3), (3, 5, "alpha", "mixed", 4, 2)])
+def test_coarse_top_switch(dim, depth, coef, precision, default, top, monkeypatch):
+    """BMG_COARSE_TOP moves the level up to which a cycle runs in one
+    workgroup, also beyond what k_coarse_rb takes, with the same values."""
+    print("block coarse top", dim, depth, coef, precision, top, flush=True)
+    out = []
+    for t in (None, top):
+        monkeypatch.delenv("BMG_COARSE_TOP", raising=False)
+        if t is not None:
+            monkeypatch.setenv("BMG_COARSE_TOP", str(t))
+        g = _grid(dim, depth, "walls", coef, precision)
+        g.residual()
+        g.mg_cycle(4, 0)
+        g.profile(True)
+        g.mg_cycle(4, 0)
+        g.synchronize()
+        assert g.profile_get("relax_coarse")[1] == _coarse_launches(dim, depth, default if t is None else t, 4)
+        out.append((g.residual(), g.get_a()))
+    assert out[0][0] == out[1][0] and np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("threads", [64, 320])
+def test_coarse_block_switch(threads, monkeypatch):
+    """BMG_COARSE_BLOCK takes the coarse kernel whose threads it sets: on a
+    grid that ends there the correction is then a launch of its own."""
+    print("block coarse threads", threads, flush=True)
+    out = []
+    for t in (None, threads):
+        if t is not None:
+            monkeypatch.setenv("BMG_COARSE_BLOCK", str(t))
+        g = _grid(2, 5, "channel", "alpha lam", "fp64")
+        g.residual()
+        g.profile(True)
+        g.mg_cycle(3, 0)
+        g.synchronize()
+        assert g.profile_get("correction")[1] == (0 if t is None else 1)
+        out.append((g.residual(), g.get_a()))
+    assert out[0][0] == out[1][0] and np.array_equal(out[0][1], out[1][1])
