@@ -30,7 +30,7 @@ F_A, F_B, F_RES, F_DA, F_LAMBDA, F_ALPHA = range(6)
 F_S = 8  # trees: user scalar k is F_S + k, k < USER_SCALARS (adapt_wavelet's scalars)
 USER_SCALARS = 4
 PROFILE_KINDS = {"relax_fine": 0, "residual": 1, "restriction": 2,
-                 "prolongation": 3, "correction": 4, "relax_coarse": 5, "relax_fine2": 6}
+                 "prolongation": 3, "correction": 4, "relax_coarse": 5, "relax_fine2": 6, "relax_fine_tile": 7}
 
 # every symbol declared in include/bmg.h
 EXPORTS = [

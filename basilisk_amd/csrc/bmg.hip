@@ -76,6 +76,7 @@ enum {
   PROF_CORRECT,
   PROF_RELAX_COARSE,
   PROF_RELAX_FINE2,
+  PROF_RELAX_TILE,
   PROF_N
 };
 
@@ -1113,7 +1114,7 @@ int tile_sweep(bmg_grid* g, int l, int ns, int src, int dst, bool correct) {
                        src < 0 ? (const T*)g->L[l - 1].da[0] : nullptr, (T*)lv.da[dst], correct ? g->a : nullptr,
                        (const T*)lv.res, k, geo, bc, bcc, (T)(D * D), A);
   };
-  ProfScope ps(g, l == g->depth ? PROF_RELAX_FINE : PROF_RELAX_COARSE);
+  ProfScope ps(g, l == g->depth ? PROF_RELAX_TILE : PROF_RELAX_COARSE);
   const bool af = k.lo[0] != nullptr;
   [[maybe_unused]] const int v = tile_variant<DIM>(lv.n);
   if constexpr (DIM == 2) {

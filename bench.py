@@ -259,7 +259,7 @@ def run_precision(bmg, torch, prob, prec, args):
     st = solve_once(g, zeros, tol)
     kinds = {}
     for k in ("relax_fine", "residual", "restriction", "prolongation", "correction", "relax_coarse",
-              "relax_fine2"):
+              "relax_fine2", "relax_fine_tile"):
         ms, n = g.profile_get(k)
         kinds[k] = {"ms": ms, "count": n}
     g.profile(False)
@@ -567,7 +567,8 @@ def main():
         am = am - am.mean()
         line["mixed_vs_fp64_rel_maxnorm"] = float(np.abs(am - af).max() / np.abs(af).max())
         pf = f["profile"]["relax_fine"]
-        line["fp64_sweep_gbs"] = round(6 * 8 * N / (pf["ms"] / max(pf["count"], 1) * 1e-3) / 1e9, 1)
+        if pf["count"]:  # (grids up to 64^3 sweep by tiles, several sweeps per launch)
+            line["fp64_sweep_gbs"] = round(6 * 8 * N / (pf["ms"] / pf["count"] * 1e-3) / 1e9, 1)
     line["kernel_ms"] = {k: round(v["ms"], 3) for k, v in r["profile"].items()}
     if r.get("project"):
         # project() (poisson.h:469-509) of the config's face velocity: the

@@ -284,7 +284,14 @@ int bmg_coef_gradient(bmg_grid *g, const double *psi, double *galpha_x, double *
    relax (one sweep per launch), 1 = residual, 2 = restriction,
    3 = prolongation, 4 = correction, 5 = coarse-level relax, 6 = fine-level
    relax of the two-sweep kernel (two sweeps per launch; FP32 levels of
-   256^3 cells and more) */
+   256^3 cells and more), 7 = fine-level relax by tiles (up to 4 sweeps per
+   launch in 2D, 2 in 3D, with the prolongation to that level and, where the
+   cycle corrects by itself, the correction; 2D levels of 64^2 cells and
+   more, 3D ones of up to 64^3).  Kind 5 counts launches of all levels below
+   the finest: one for the coarsest levels together, with the restrictions
+   and prolongations between them (and the correction of a grid that ends
+   there), and on the levels above several sweeps where kinds 6 or 7 would
+   be the finest level's. */
 int bmg_profile_enable(bmg_grid *g, int enable);
 int bmg_profile_get(bmg_grid *g, int kind, double *total_ms, long *count);
 

@@ -160,3 +160,23 @@ def test_coarse_block_switch(threads, monkeypatch):
         assert g.profile_get("correction")[1] == (0 if t is None else 1)
         out.append((g.residual(), g.get_a()))
     assert out[0][0] == out[1][0] and np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("dim,depth,kernel,kind,launches",
+                         [(2, 7, None, "relax_fine_tile", 2), (3, 5, None, "relax_fine_tile", 3),
+                          (2, 7, "inplace", "relax_fine", 5), (3, 7, None, "relax_fine", 5)])
+def test_profile_kinds_of_the_finest_level(dim, depth, kernel, kind, launches, monkeypatch):
+    """relax_fine counts launches of one sweep; tiles, which run several and
+    interpolate and correct as well, are a kind of their own."""
+    print("block profile", dim, depth, kernel, flush=True)
+    if kernel:
+        monkeypatch.setenv("BMG_RB_KERNEL", kernel)
+    g = _grid(dim, depth, "walls", "", "fp64")
+    g.residual()
+    g.profile(True)
+    g.mg_cycle(5, 0)
+    g.synchronize()
+    count = {k: g.profile_get(k)[1] for k in bmg.PROFILE_KINDS}
+    fine = {k: count[k] for k in ("relax_fine", "relax_fine2", "relax_fine_tile")}
+    assert fine == dict.fromkeys(fine, 0) | {kind: launches}
+    assert count["correction"] == (0 if kind == "relax_fine_tile" else 1)
