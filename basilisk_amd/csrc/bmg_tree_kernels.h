@@ -118,7 +118,7 @@ __global__ __launch_bounds__(kB) void k_t_box(const BoxRule* __restrict__ R, int
 
 // An entry of the parent rings and of the colour lists' neighbour rows: a
 // slot, or ~r for the ghost cell that box rule r fills.  A reader either
-// takes the ghost's stored value (GhostStored, after the box pass of that
+// takes the ghost's stored value (t_ring_stored, after the box pass of that
 // level) or evaluates the rule itself (GhostRule), which gives the value
 // that a box pass just before the read would have stored: the cycle does
 // the latter and runs no box pass at all.  A tree cycle is bound by the
@@ -127,12 +127,6 @@ __global__ __launch_bounds__(kB) void k_t_box(const BoxRule* __restrict__ R, int
 // restricted and interpolated, a relax of the finest level of a quadtree of
 // levels 5-11 (225k leaves) takes 4 launches instead of 20: FP64 solve 44.6
 // -> 25.4 ms; octree of levels 4-8 (0.58M leaves), mixed, 26.3 -> 17.1 ms.
-template <typename T>
-struct GhostStored {
-  const T* f;
-  const BoxRule* box;
-  __device__ __forceinline__ T operator()(int v) const { return f[v >= 0 ? v : box[~v].ghost]; }
-};
 template <typename T>
 struct GhostRule {
   const T* f;
@@ -195,16 +189,16 @@ __global__ __launch_bounds__(kB) void k_t_restrict_tree(RestrictLevels L, const 
 }
 
 // bilinear (grid/multigrid-common.h:124-140) of child m (foreach_child
-// order) of a record, from its 3^dim ring g read through `at`
+// order) of a record; at(p) is the value at place p of its 3^dim ring
 template <typename T, int DIM, typename L>
-__device__ __forceinline__ T t_bilinear_child(const int* __restrict__ g, int m, const L& at) {
+__device__ __forceinline__ T t_bilinear_child(int m, const L& at) {
   if (DIM == 2) {
     const int cx = 2 * (m >> 1) - 1, cy = 2 * (m & 1) - 1;
-    T c0 = at(g[4]), c1 = at(g[(1 + cx) * 3 + 1]), c2 = at(g[3 + 1 + cy]), c3 = at(g[(1 + cx) * 3 + 1 + cy]);
+    T c0 = at(4), c1 = at((1 + cx) * 3 + 1), c2 = at(3 + 1 + cy), c3 = at((1 + cx) * 3 + 1 + cy);
     return (T(9) * c0 + T(3) * (c1 + c2) + c3) / T(16);
   } else {
     const int cx = 2 * (m >> 2) - 1, cy = 2 * ((m >> 1) & 1) - 1, cz = 2 * (m & 1) - 1;
-#define RG(x, y, z) at(g[((1 + (x)) * 3 + 1 + (y)) * 3 + 1 + (z)])
+#define RG(x, y, z) at(((1 + (x)) * 3 + 1 + (y)) * 3 + 1 + (z))
     T c000 = RG(0, 0, 0), c100 = RG(cx, 0, 0), c010 = RG(0, cy, 0), c001 = RG(0, 0, cz);
     T c110 = RG(cx, cy, 0), c101 = RG(cx, 0, cz), c011 = RG(0, cy, cz), c111 = RG(cx, cy, cz);
 #undef RG
@@ -212,11 +206,34 @@ __device__ __forceinline__ T t_bilinear_child(const int* __restrict__ g, int m, 
   }
 }
 
-// the 2^dim children of a record
-template <typename T, int DIM, typename L>
-__device__ __forceinline__ void t_bilinear_children(const int* __restrict__ g, const L& at, T* v) {
+// the ring g of a record, with the ghosts stored in f.  Every entry is read
+// once, all slots before all values: the children read 4 or 8 entries each,
+// and a ghost resolved at each of these reads was a chain of loads apiece and
+// took the registers (FP64 octree of 36k leaves: k_t_prolong 13.5 us a launch,
+// now 3.8; k_t_wavelet, at half the waves, 10.2, now 3.6; k_t_ops, which
+// spilled, 23, now 11).
+template <typename T, int DIM>
+__device__ __forceinline__ void t_ring_stored(const int* __restrict__ g, const T* f, const BoxRule* box, T* r) {
+  constexpr int NR = DIM == 2 ? 9 : 27;
+  int s[NR], any = 0;
 #pragma unroll
-  for (int m = 0; m < (1 << DIM); m++) v[m] = t_bilinear_child<T, DIM>(g, m, at);
+  for (int m = 0; m < NR; m++) any |= s[m] = g[m];
+  if (any < 0) {
+#pragma unroll
+    for (int m = 0; m < NR; m++)
+      if (s[m] < 0) s[m] = box[~s[m]].ghost;
+  }
+#pragma unroll
+  for (int m = 0; m < NR; m++) r[m] = f[s[m]];
+}
+
+// the 2^dim children of a record, the ghosts of its ring stored in f
+template <typename T, int DIM>
+__device__ __forceinline__ void t_bilinear_children(const int* __restrict__ g, const T* f, const BoxRule* box, T* v) {
+  T r[DIM == 2 ? 9 : 27];
+  t_ring_stored<T, DIM>(g, f, box, r);
+#pragma unroll
+  for (int m = 0; m < (1 << DIM); m++) v[m] = t_bilinear_child<T, DIM>(m, [&](int p) { return r[p]; });
 }
 
 // bilinear into the 2^dim children of each record from its 3^dim ring, with
@@ -224,7 +241,7 @@ __device__ __forceinline__ void t_bilinear_children(const int* __restrict__ g, c
 template <typename T, int DIM>
 __device__ __forceinline__ void t_prolong_one(const int* __restrict__ g, int child0, T* f, const BoxRule* box) {
   T v[1 << DIM];
-  t_bilinear_children<T, DIM>(g, GhostStored<T>{f, box}, v);
+  t_bilinear_children<T, DIM>(g, f, box, v);
 #pragma unroll
   for (int m = 0; m < (1 << DIM); m++) f[child0 + m] = v[m];
 }
@@ -247,7 +264,9 @@ __device__ __forceinline__ void t_child_one(int item, const int* __restrict__ ri
                                             T* f, const BoxRule* box, const BCT& bc, int bk, double L0) {
   constexpr int NR = DIM == 2 ? 9 : 27;
   const int r = item >> DIM, m = item & ((1 << DIM) - 1);
-  f[child0[r] + m] = t_bilinear_child<T, DIM>(ring + (size_t)r * NR, m, GhostRule<T>{f, box, bc, bk, L0});
+  const int* g = ring + (size_t)r * NR;
+  const GhostRule<T> at{f, box, bc, bk, L0};
+  f[child0[r] + m] = t_bilinear_child<T, DIM>(m, [&](int p) { return at(g[p]); });
 }
 
 template <typename T, int DIM>
@@ -763,7 +782,7 @@ __global__ __launch_bounds__(kB) void k_t_wavelet(const int* __restrict__ ring, 
   if (r >= n) return;
   constexpr int NR = DIM == 2 ? 9 : 27;
   double v[1 << DIM];
-  t_bilinear_children<double, DIM>(ring + (size_t)r * NR, GhostStored<double>{f, box}, v);
+  t_bilinear_children<double, DIM>(ring + (size_t)r * NR, f, box, v);
   const int c0 = child0[r];
 #pragma unroll
   for (int m = 0; m < (1 << DIM); m++) err[c0 + m] = fabs(f[c0 + m] - v[m]);
@@ -789,7 +808,7 @@ __global__ __launch_bounds__(kB) void k_t_refine_remap(const int* __restrict__ r
   if (r >= n) return;
   constexpr int NR = DIM == 2 ? 9 : 27;
   double v[1 << DIM];
-  t_bilinear_children<double, DIM>(ring + (size_t)r * NR, GhostStored<double>{old, nullptr}, v);
+  t_bilinear_children<double, DIM>(ring + (size_t)r * NR, old, nullptr, v);
   const int c0 = child0[r];
 #pragma unroll
   for (int m = 0; m < (1 << DIM); m++) out[c0 + m] = v[m];
