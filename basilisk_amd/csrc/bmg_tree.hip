@@ -1694,10 +1694,15 @@ int compile(bmg_tree* t) {
           return;
         }
         const size_t ai = (size_t)x.abase[m] + (gs - x.off[m]);
-        for (int k = 0; k < 2 * dim; k++) cnb[e * 2 * dim + k] = entry(m, nbr[ai * 2 * dim + k]);
+        for (int k = 0; k < 2 * dim; k++) {
+          const int v = cnb[e * 2 * dim + k] = entry(m, nbr[ai * 2 * dim + k]);
+          // relax takes a ghost's source to be the cell itself
+          if (v < 0 && (box[~v].nterm != 1 || box[~v].src != gs)) bad = true;
+        }
       }
     });
-    if (bad) return bmg::fail(BMG_ERR_ARG, "tree: colour list entry outside the active cells");
+    if (bad)
+      return bmg::fail(BMG_ERR_ARG, "tree: colour list entry outside the active cells, or a ghost with another source");
     TRY(upload(&x.col_nbr, cnb));
   }
   TRY(upload(&x.box, box));
@@ -1934,18 +1939,20 @@ int relax(bmg_tree* t, int l) {
   if (t->smoother == BMG_RELAX_JACOBI) {
     {
       TProf tp(t, seg_cells(S));
-      k_t_relax<T, DIM><<<nbk, kB, 0, t->stream>>>(S, da, F<T>(t->tmp), res, x.nbr, x.box, bct(t), t->L0, k);
+      k_t_relax<T, DIM><<<nbk, kB, 0, t->stream>>>(S, da, F<T>(t->tmp), res, x.nbr, x.box, bct(t), k);
     }
     k_t_jacobi<T><<<nbk, kB, 0, t->stream>>>(S, da, F<T>(t->tmp));
   } else if (t->smoother == BMG_RELAX_RBGS) {
     for (int c = 0; c < 2; c++) {
-      // (the stored ghosts, which a Jacobi relax may read next)
-      if (c) for (int m = 0; m <= l; m++) box<T>(t, da, BK_HOM, m);
+      // the stored ghosts, which a Jacobi relax may read next (their sources
+      // are cells of the box: every level in one launch)
+      const int ng = x.box_off[l] + x.box_n[l];
+      if (c && ng) k_t_box<T><<<nb_(ng), kB, 0, t->stream>>>(x.box, ng, da, bct(t), BK_HOM, t->L0);
       Segs SC = level_or_leaf_colour(t, l, c);
       unsigned nbc = (unsigned)SC.first_block[SC.n];
       if (nbc) {
         TProf tp(t, seg_cells(SC));
-        k_t_relax<T, DIM><<<nbc, kB, 0, t->stream>>>(SC, da, nullptr, res, x.nbr, x.box, bct(t), t->L0, k);
+        k_t_relax<T, DIM><<<nbc, kB, 0, t->stream>>>(SC, da, nullptr, res, x.nbr, x.box, bct(t), k);
       }
     }
   } else
@@ -2154,7 +2161,7 @@ struct Batcher {
       unsigned nbc = (unsigned)SC.first_block[SC.n];
       if (!nbc) continue;
       TProf tp(t, seg_cells(SC));
-      k_t_relax<T, DIM><<<nbc, kB, 0, t->stream>>>(SC, da, jac ? A.fld[2] : nullptr, A.res, x.nbr, x.box, A.bc, t->L0,
+      k_t_relax<T, DIM><<<nbc, kB, 0, t->stream>>>(SC, da, jac ? A.fld[2] : nullptr, A.res, x.nbr, x.box, A.bc,
                                                    A.k);
     }
     if (jac) {

@@ -258,3 +258,60 @@ def test_relax_after_cycle_sees_its_boundary(smoother):
     t[0].relax(7)
     t[1].mg_cycle(4, 7, 7)
     assert np.array_equal(t[0].get_da(), t[1].get_da())
+
+
+SIDES = [bmg.BC_DIRICHLET, bmg.BC_NEUMANN, bmg.BC_SYMMETRY, bmg.BC_DIRICHLET, bmg.BC_NEUMANN, bmg.BC_DIRICHLET]
+
+
+def _numpy_relax(da, res, lam, ghosts, D, cells, jacobi):
+    """One pass of relax (poisson.h:303-320) with alpha = 1 over `cells` of a
+    full level; the ghost across a wall is +-ghosts of the cell itself."""
+    n, d = -(D * D) * res, -lam * (D * D) * np.ones_like(da)
+    for c in range(da.ndim):
+        nb = []
+        for side, step in ((2 * c, 1), (2 * c + 1, -1)):  # above, below
+            v = np.roll(da, -step, c)
+            wall = [slice(None)] * da.ndim
+            wall[c] = -1 if step == 1 else 0
+            v[tuple(wall)] = (-1.0 if SIDES[side] == bmg.BC_DIRICHLET else 1.0) * ghosts[tuple(wall)]
+            nb.append(v)
+        n = n + (1.0 * nb[0] + 1.0 * nb[1])
+        d = d + (1.0 + 1.0)
+    w = n / d
+    return np.where(cells, (da + 2.0 * w) / 3.0 if jacobi else w, da)
+
+
+@pytest.mark.parametrize("dim,depth", [(2, 1), (2, 3), (2, 6), (3, 1), (3, 2), (3, 4)])
+def test_relax_reads_ghosts_of_every_side(dim, depth):
+    """relax() on a full level with homogeneous Dirichlet, Neumann and
+    symmetric sides, bit for bit: red-black evaluates the ghosts, a Jacobi
+    relax after it reads the values stored between the colours."""
+    print("relax ghosts", dim, depth, flush=True)
+    g = bmg.Tree(dim, 1.0, (0.0, 0.0, 0.0), smoother="rbgs")
+    g.refine(lambda x, y, z, lev: lev < depth)
+    n = 1 << depth
+    _, xyz = g.leaves()
+    at = tuple((xyz[:, c] * n).astype(int) for c in range(dim))
+    rng = np.random.default_rng(dim * 10 + depth)
+    b = rng.standard_normal((n,) * dim)
+    g.set_b(b[at].copy())
+    g.set_a(np.zeros(len(xyz)))
+    g.set_lambda(-1.25)
+    for side in range(2 * dim):
+        g.set_bc(side, SIDES[side])
+    g.residual()
+    res = np.empty_like(b)
+    res[at] = g.get_res()
+    D, da = 1.0 / n, np.zeros_like(b)
+    g.mg_cycle(0, depth, depth)  # da = 0
+    parity = np.indices(b.shape).sum(0) & 1
+    for _ in range(3):
+        g.relax(depth)
+        da = _numpy_relax(da, res, -1.25, da, D, parity == 0, False)
+        ghosts = da.copy()
+        da = _numpy_relax(da, res, -1.25, da, D, parity == 1, False)
+        assert np.array_equal(g.get_da(), da[at])
+    g.set_smoother("jacobi")
+    g.relax(depth)
+    da = _numpy_relax(da, res, -1.25, ghosts, D, parity >= 0, True)
+    assert np.array_equal(g.get_da(), da[at])
