@@ -705,7 +705,7 @@ struct DevIndex {
   // the halo cells that relax, the initial guesses and the residual's faces
   // read, as 2^dim * record + child, by dependency stage (a cell interpolated
   // from halo cells of stage k - 1 has stage k) and then by level
-  int* halo = nullptr;
+  int* halo = nullptr;        // (halo_end_d and drec follow in the same array)
   int* halo_end_d = nullptr;
   int nstage = 0;
   std::vector<int> halo_end;  // [stage * (depth + 1) + level]: end of the stage's cells up to that level
@@ -886,8 +886,9 @@ void free_device(bmg_tree* t) {
   drop_graphs(t);
   DevIndex& x = t->ix;
   for (void* p : {(void*)x.nbr, (void*)x.rec_self, (void*)x.rec_child0, (void*)x.rec_ring, (void*)x.colour,
-                  (void*)x.leaf_gs, (void*)x.lvl_leaves, (void*)x.col_list, (void*)x.col_nbr, (void*)x.halo, (void*)x.halo_end_d, (void*)x.drec, (void*)x.box, (void*)x.fops, (void*)x.hf, (void*)x.fr,
-                  (void*)x.fp, (void*)x.fc, (void*)x.fv_gs, (void*)x.fv_d, (void*)x.fc_tmp, (void*)x.lvinfo})
+                  (void*)x.leaf_gs, (void*)x.lvl_leaves, (void*)x.col_list, (void*)x.col_nbr, (void*)x.halo,
+                  (void*)x.box, (void*)x.fops, (void*)x.hf, (void*)x.fr, (void*)x.fp, (void*)x.fc, (void*)x.fv_gs,
+                  (void*)x.fv_d, (void*)x.fc_tmp, (void*)x.lvinfo})
     dfree_(p);
   x = DevIndex();
   bool mixed = t->precision == BMG_MIXED;
@@ -1095,100 +1096,6 @@ int compile(bmg_tree* t) {
     return v;
   };
   clk.mark("compile: slots");
-  // active neighbours and colours
-  long NA = x.abase[D] + x.nA[D];
-  table<int> nbr((size_t)NA * 2 * dim);
-  table<uint8_t> colour(NA);
-  for (int l = 0; l <= D; l++)
-    par_for((size_t)x.nA[l], [&](size_t q0, size_t q1) {
-      for (size_t q = q0; q < q1; q++) {
-        IJK c = T.active[l][q];
-        size_t ai = (size_t)x.abase[l] + q;
-        for (int d = 0; d < dim; d++) {
-          int o[3] = {0, 0, 0};
-          o[d] = 1;
-          nbr[ai * 2 * dim + 2 * d] = chk(S(l, c.i - o[0], c.j - o[1], c.k - o[2]));
-          nbr[ai * 2 * dim + 2 * d + 1] = chk(S(l, c.i + o[0], c.j + o[1], c.k + o[2]));
-        }
-        colour[ai] = (uint8_t)((c.i + c.j + c.k) & 1);
-      }
-    });
-  if (!ok) return bmg::fail(BMG_ERR_ARG, "tree: active cell without neighbours");
-  // the non-leaf active cells of each level (indices into active[l])
-  clk.mark("compile: tables: neighbours");
-  std::vector<std::vector<int>> nonleaf(D + 1);
-  for (int l = 0; l <= D; l++) {
-    std::vector<uint8_t> isnl((size_t)x.nA[l]);
-    par_for((size_t)x.nA[l], [&](size_t q0, size_t q1) {
-      for (size_t q = q0; q < q1; q++) {
-        const IJK& c = T.active[l][q];
-        isnl[q] = !T.is_leaf(*T.L[l].find(c.i, c.j, c.k));
-      }
-    });
-    for (int q = 0; q < x.nA[l]; q++)
-      if (isnl[q]) nonleaf[l].push_back(q);
-  }
-  // parent records: non-leaf active cells, then prolongation leaves
-  const int NR = dim == 3 ? 27 : 9;
-  x.rec_off.assign(D + 1, 0);
-  x.n_nonleaf.assign(D + 1, 0);
-  x.n_prolong.assign(D + 1, 0);
-  size_t nrec = 0;
-  for (int l = 0; l <= D; l++) {
-    x.rec_off[l] = (int)nrec;
-    x.n_nonleaf[l] = (int)nonleaf[l].size();
-    x.n_prolong[l] = (int)T.prolong[l].size();
-    nrec += (size_t)x.n_nonleaf[l] + x.n_prolong[l];
-  }
-  table<int> rself(nrec), rchild(nrec), rring(nrec * NR);
-  auto add_rec = [&](size_t r, int l, IJK c) {
-    rself[r] = chk(S(l, c.i, c.j, c.k));
-    int c0 = chk(S(l + 1, 2 * c.i - GH, 2 * c.j - GH, dim == 3 ? 2 * c.k - GH : 0));
-    rchild[r] = c0;
-    // the kernels address the children as child0 + (foreach_child index)
-    int m = 0;
-    for (int a = 0; a < 2; a++)
-      for (int b = 0; b < 2; b++)
-        for (int e = 0; e < T.kext(); e++, m++)
-          if (S(l + 1, 2 * c.i - GH + a, 2 * c.j - GH + b, dim == 3 ? 2 * c.k - GH + e : 0) != c0 + m)
-            ok.store(false, std::memory_order_relaxed);
-    int e0 = dim == 3 ? -1 : 0, e1 = dim == 3 ? 1 : 0;
-    size_t w = r * NR;
-    for (int a = -1; a <= 1; a++)
-      for (int b = -1; b <= 1; b++)
-        for (int e = e0; e <= e1; e++) rring[w++] = chk(S(l, c.i + a, c.j + b, c.k + e));
-  };
-  for (int l = 0; l <= D; l++) {
-    const size_t r0 = x.rec_off[l], np = x.n_nonleaf[l];
-    par_for(np, [&](size_t k0, size_t k1) {
-      for (size_t k = k0; k < k1; k++) add_rec(r0 + k, l, T.active[l][nonleaf[l][k]]);
-    });
-    par_for(T.prolong[l].size(), [&](size_t k0, size_t k1) {
-      for (size_t k = k0; k < k1; k++) add_rec(r0 + np + k, l, T.prolong[l][k]);
-    });
-  }
-  if (!ok) return bmg::fail(BMG_ERR_ARG, "tree: parent record with an unallocated ring");
-  // leaves: global cache order and per level
-  x.nleaf = (long)T.leaf_c.size();
-  clk.mark("compile: tables: parent records");
-  table<int> leaf_gs(x.nleaf);
-  std::vector<std::vector<int>> lv(D + 1);
-  par_for((size_t)x.nleaf, [&](size_t n0, size_t n1) {
-    for (size_t n = n0; n < n1; n++) {
-      IJK c = T.leaf_c[n];
-      leaf_gs[n] = chk(S(T.leaf_level[n], c.i, c.j, c.k));
-    }
-  });
-  for (long n = 0; n < x.nleaf; n++) lv[T.leaf_level[n]].push_back(leaf_gs[n]);
-  std::vector<int> lvl_leaves;
-  x.leaf_off.assign(D + 1, 0);
-  x.leaf_n.assign(D + 1, 0);
-  for (int l = 0; l <= D; l++) {
-    x.leaf_off[l] = (int)lvl_leaves.size();
-    x.leaf_n[l] = (int)lv[l].size();
-    lvl_leaves.insert(lvl_leaves.end(), lv[l].begin(), lv[l].end());
-  }
-  clk.mark("compile: tables: leaves");
   // box rules (boundary cache order)
   x.bc_off.assign(D + 2, 0);
   for (int l = 0; l <= D; l++) {
@@ -1269,6 +1176,152 @@ int compile(bmg_tree* t) {
     x.box_n[l] = (int)box.size() - x.box_off[l];
   }
   clk.mark("compile: tables: box rules");
+  // the non-leaf active cells of each level (indices into active[l])
+  std::vector<std::vector<int>> nonleaf(D + 1);
+  for (int l = 0; l <= D; l++) {
+    std::vector<uint8_t> isnl((size_t)x.nA[l]);
+    par_for((size_t)x.nA[l], [&](size_t q0, size_t q1) {
+      for (size_t q = q0; q < q1; q++) {
+        const IJK& c = T.active[l][q];
+        isnl[q] = !T.is_leaf(*T.L[l].find(c.i, c.j, c.k));
+      }
+    });
+    for (int q = 0; q < x.nA[l]; q++)
+      if (isnl[q]) nonleaf[l].push_back(q);
+  }
+  // parent records: non-leaf active cells, then prolongation leaves
+  const int NR = dim == 3 ? 27 : 9;
+  x.rec_off.assign(D + 1, 0);
+  x.n_nonleaf.assign(D + 1, 0);
+  x.n_prolong.assign(D + 1, 0);
+  size_t nrec = 0;
+  for (int l = 0; l <= D; l++) {
+    x.rec_off[l] = (int)nrec;
+    x.n_nonleaf[l] = (int)nonleaf[l].size();
+    x.n_prolong[l] = (int)T.prolong[l].size();
+    nrec += (size_t)x.n_nonleaf[l] + x.n_prolong[l];
+  }
+  // the parent rings and the colour lists' neighbour rows name a ghost of the
+  // box by its rule (~r), see GhostRule
+  if (nrec * (size_t)nch > (size_t)INT_MAX) return bmg::fail(BMG_ERR_UNSUPPORTED, "tree: too many parent records");
+  std::vector<int> gbase(D + 1), hbase(D + 1);
+  std::vector<std::vector<int>> rule(D + 1);
+  std::vector<size_t> hoff(D + 2, 0);
+  for (int l = 0; l <= D; l++) {
+    hbase[l] = x.off[l] + x.nA[l];
+    gbase[l] = hbase[l] + (l ? nch * x.n_prolong[l - 1] : 0);
+    hoff[l + 1] = hoff[l] + (size_t)(gbase[l] - hbase[l]);
+    rule[l].assign((size_t)((l < D ? x.off[l + 1] : (int)NS) - gbase[l]), -1);
+    for (int r = x.box_off[l]; r < x.box_off[l] + x.box_n[l]; r++)
+      if (box[r].ghost >= gbase[l] && box[r].ghost - gbase[l] < (int)rule[l].size())
+        rule[l][box[r].ghost - gbase[l]] = r;
+  }
+  auto entry = [&](int l, int v) {
+    if (v < gbase[l] || v - gbase[l] >= (int)rule[l].size()) return v;
+    const int r = rule[l][v - gbase[l]];
+    return r >= 0 ? ~r : v;
+  };
+  // The halo cells that a table's entries read are marked as the entries are
+  // made (0: not read; 1: read; later the stage).  Most entries name active
+  // cells, which come before the others of their level: one comparison.
+  std::vector<uint8_t> stage(hoff[D + 1], 0);
+  // the halo cell an entry of level l reads: its index, or -1
+  auto halo_of = [&](int l, int v) -> long {
+    if (v < 0) v = box[~v].nterm ? box[~v].src : -1;
+    return v >= hbase[l] && v < gbase[l] ? (long)(hoff[l] + (size_t)(v - hbase[l])) : -1;
+  };
+  auto mark = [&](int l, int v) {
+    const long h = halo_of(l, v);
+    if (h >= 0) __atomic_store_n(&stage[(size_t)h], (uint8_t)1, __ATOMIC_RELAXED);
+  };
+  auto reads = [&](int l, int slot) {
+    if (slot >= hbase[l]) mark(l, entry(l, slot));
+    return slot;
+  };
+  // active neighbours and colours
+  long NA = x.abase[D] + x.nA[D];
+  table<int> nbr((size_t)NA * 2 * dim);
+  table<uint8_t> colour(NA);
+  for (int l = 0; l <= D; l++)
+    par_for((size_t)x.nA[l], [&](size_t q0, size_t q1) {
+      for (size_t q = q0; q < q1; q++) {
+        IJK c = T.active[l][q];
+        size_t ai = (size_t)x.abase[l] + q;
+        for (int d = 0; d < dim; d++) {
+          int o[3] = {0, 0, 0};
+          o[d] = 1;
+          nbr[ai * 2 * dim + 2 * d] = reads(l, chk(S(l, c.i - o[0], c.j - o[1], c.k - o[2])));
+          nbr[ai * 2 * dim + 2 * d + 1] = reads(l, chk(S(l, c.i + o[0], c.j + o[1], c.k + o[2])));
+        }
+        colour[ai] = (uint8_t)((c.i + c.j + c.k) & 1);
+      }
+    });
+  if (!ok) return bmg::fail(BMG_ERR_ARG, "tree: active cell without neighbours");
+  clk.mark("compile: tables: neighbours");
+  table<int> rself(nrec), rchild(nrec), rring(nrec * NR);
+  // the children of nonleaf record k of a level are active cells nch k ..
+  // of the next one
+  std::atomic<bool> ordered{true};
+  // (the rings of the prolongation leaves are read by halo cells only, which
+  // the closure below marks)
+  auto add_rec = [&](size_t r, int l, IJK c, bool read) {
+    rself[r] = chk(S(l, c.i, c.j, c.k));
+    int c0 = chk(S(l + 1, 2 * c.i - GH, 2 * c.j - GH, dim == 3 ? 2 * c.k - GH : 0));
+    rchild[r] = c0;
+    // the kernels address the children as child0 + (foreach_child index)
+    int m = 0;
+    for (int a = 0; a < 2; a++)
+      for (int b = 0; b < 2; b++)
+        for (int e = 0; e < T.kext(); e++, m++)
+          if (S(l + 1, 2 * c.i - GH + a, 2 * c.j - GH + b, dim == 3 ? 2 * c.k - GH + e : 0) != c0 + m)
+            ok.store(false, std::memory_order_relaxed);
+    int e0 = dim == 3 ? -1 : 0, e1 = dim == 3 ? 1 : 0;
+    size_t w = r * NR;
+    for (int a = -1; a <= 1; a++)
+      for (int b = -1; b <= 1; b++)
+        for (int e = e0; e <= e1; e++) {
+          int v = chk(S(l, c.i + a, c.j + b, c.k + e));
+          if (v >= hbase[l]) {
+            v = entry(l, v);
+            if (read) mark(l, v);
+          }
+          rring[w++] = v;
+        }
+  };
+  for (int l = 0; l <= D; l++) {
+    const size_t r0 = x.rec_off[l], np = x.n_nonleaf[l];
+    par_for(np, [&](size_t k0, size_t k1) {
+      for (size_t k = k0; k < k1; k++) {
+        add_rec(r0 + k, l, T.active[l][nonleaf[l][k]], true);
+        if (rchild[r0 + k] != x.off[l + 1] + (int)k * nch) ordered.store(false, std::memory_order_relaxed);
+      }
+    });
+    par_for(T.prolong[l].size(), [&](size_t k0, size_t k1) {
+      for (size_t k = k0; k < k1; k++) add_rec(r0 + np + k, l, T.prolong[l][k], false);
+    });
+  }
+  if (!ok) return bmg::fail(BMG_ERR_ARG, "tree: parent record with an unallocated ring");
+  // leaves: global cache order and per level
+  x.nleaf = (long)T.leaf_c.size();
+  clk.mark("compile: tables: parent records");
+  table<int> leaf_gs(x.nleaf);
+  std::vector<std::vector<int>> lv(D + 1);
+  par_for((size_t)x.nleaf, [&](size_t n0, size_t n1) {
+    for (size_t n = n0; n < n1; n++) {
+      IJK c = T.leaf_c[n];
+      leaf_gs[n] = chk(S(T.leaf_level[n], c.i, c.j, c.k));
+    }
+  });
+  for (long n = 0; n < x.nleaf; n++) lv[T.leaf_level[n]].push_back(leaf_gs[n]);
+  std::vector<int> lvl_leaves;
+  x.leaf_off.assign(D + 1, 0);
+  x.leaf_n.assign(D + 1, 0);
+  for (int l = 0; l <= D; l++) {
+    x.leaf_off[l] = (int)lvl_leaves.size();
+    x.leaf_n[l] = (int)lv[l].size();
+    lvl_leaves.insert(lvl_leaves.end(), lv[l].begin(), lv[l].end());
+  }
+  clk.mark("compile: tables: leaves");
   // residual face ops per level, and the face-cache value map (entry order
   // then dimension); the positions come from prefix counts of the flag bits
   const size_t NF = T.faces.size();
@@ -1303,7 +1356,7 @@ int compile(bmg_tree* t) {
         if (f.flags & (1 << d)) {
           int m[3] = {fc[0], fc[1], fc[2]};
           m[d]--;
-          FaceOp op = {chk(S(l, fc[0], fc[1], fc[2])), chk(S(l, m[0], m[1], m[2])), d};
+          FaceOp op = {reads(l, chk(S(l, fc[0], fc[1], fc[2]))), reads(l, chk(S(l, m[0], m[1], m[2]))), d};
           fops[lp++] = op;
           fv_gs[g] = op.gs;
           fv_d[g++] = d;
@@ -1311,29 +1364,7 @@ int compile(bmg_tree* t) {
     }
   });
   clk.mark("compile: tables: face ops");
-  // ghost entries of the rings become box rules (~r), see GhostRule
-  std::vector<int> gbase(D + 1), hbase(D + 1);
-  std::vector<std::vector<int>> rule(D + 1);
-  for (int l = 0; l <= D; l++) {
-    hbase[l] = x.off[l] + x.nA[l];
-    gbase[l] = hbase[l] + (l ? nch * x.n_prolong[l - 1] : 0);
-    rule[l].assign((size_t)((l < D ? x.off[l + 1] : (int)NS) - gbase[l]), -1);
-    for (int r = x.box_off[l]; r < x.box_off[l] + x.box_n[l]; r++)
-      if (box[r].ghost >= gbase[l] && box[r].ghost - gbase[l] < (int)rule[l].size())
-        rule[l][box[r].ghost - gbase[l]] = r;
-  }
-  auto entry = [&](int l, int v) {
-    if (v < gbase[l] || v - gbase[l] >= (int)rule[l].size()) return v;
-    const int r = rule[l][v - gbase[l]];
-    return r >= 0 ? ~r : v;
-  };
-  for (int l = 0; l <= D; l++) {
-    const size_t w0 = (size_t)x.rec_off[l] * NR;
-    par_for((size_t)(x.n_nonleaf[l] + x.n_prolong[l]) * NR, [&](size_t k0, size_t k1) {
-      for (size_t k = k0; k < k1; k++) rring[w0 + k] = entry(l, rring[w0 + k]);
-    });
-  }
-  // the halo cells that anything reads, and their dependency stages
+  // the coarsest level with leaves and the uniform levels at the top
   x.lneed = D;
   for (int l = D; l >= 0; l--)
     if (x.leaf_n[l] || x.face_n[l] || x.n_prolong[l]) x.lneed = l;
@@ -1348,38 +1379,10 @@ int compile(bmg_tree* t) {
     if (!full) break;
     x.ctop = l;
   }
+  // the halo cells that anything reads (the marked ones and what they are
+  // interpolated from), and their dependency stages
   table<int> halo;
   {
-    std::vector<size_t> hoff(D + 2, 0);
-    for (int l = 0; l <= D; l++) hoff[l + 1] = hoff[l] + (size_t)(gbase[l] - hbase[l]);
-    if (nrec * (size_t)nch > (size_t)INT_MAX) return bmg::fail(BMG_ERR_UNSUPPORTED, "tree: too many parent records");
-    // 0: not read; then 1 (read), later the stage
-    std::vector<uint8_t> stage(hoff[D + 1], 0);
-    // the halo cell an entry of level l reads: its index, or -1
-    auto halo_of = [&](int l, int v) -> long {
-      if (v < 0) v = box[~v].nterm ? box[~v].src : -1;
-      return v >= hbase[l] && v < gbase[l] ? (long)(hoff[l] + (size_t)(v - hbase[l])) : -1;
-    };
-    auto mark = [&](int l, int v) {
-      const long h = halo_of(l, v);
-      if (h >= 0) __atomic_store_n(&stage[(size_t)h], (uint8_t)1, __ATOMIC_RELAXED);
-    };
-    for (int l = 0; l <= D; l++) {
-      const size_t a0 = (size_t)x.abase[l] * 2 * dim, w0 = (size_t)x.rec_off[l] * NR;
-      par_for((size_t)x.nA[l] * 2 * dim, [&](size_t k0, size_t k1) {
-        for (size_t k = k0; k < k1; k++) mark(l, entry(l, nbr[a0 + k]));
-      });
-      par_for((size_t)x.n_nonleaf[l] * NR, [&](size_t k0, size_t k1) {
-        for (size_t k = k0; k < k1; k++) mark(l, rring[w0 + k]);
-      });
-      par_for((size_t)x.face_n[l], [&](size_t k0, size_t k1) {
-        for (size_t k = k0; k < k1; k++) {
-          const FaceOp& f = fops[(size_t)x.face_off[l] + k];
-          mark(l, entry(l, f.gs));
-          mark(l, entry(l, f.gm));
-        }
-      });
-    }
     // ring position of term k of child m's interpolation
     int pos[8][8];
     for (int m = 0; m < nch; m++)
@@ -1392,8 +1395,9 @@ int compile(bmg_tree* t) {
         pos[m][k] = p;
       }
     auto terms = [&](int l, size_t h, auto&& f) {  // the ring entries halo cell h of level l is interpolated from
-      const size_t r = (size_t)x.rec_off[l - 1] + x.n_nonleaf[l - 1] + h / nch;
-      for (int k = 0; k < nch; k++) f(rring[r * NR + pos[h % nch][k]]);
+      const size_t r = (size_t)x.rec_off[l - 1] + x.n_nonleaf[l - 1] + (h >> dim);
+      const int* at = pos[h & (size_t)(nch - 1)];
+      for (int k = 0; k < nch; k++) f(rring[r * NR + at[k]]);
     };
     for (int l = D; l >= 1; l--)
       par_for(hoff[l + 1] - hoff[l], [&](size_t h0, size_t h1) {
@@ -1429,31 +1433,36 @@ int compile(bmg_tree* t) {
       for (int l = 0; l <= D; l++) x.halo_end[(size_t)k * (D + 1) + l] = end += count[l][k];
       halo.insert(halo.end(), items[k].begin(), items[k].end());
     }
-    TRY(upload(&x.halo, halo));
-    TRY(upload(&x.halo_end_d, x.halo_end));
   }
-  // the children of nonleaf record k of a level are active cells nch k ..
-  // of the next one, so its child records are a run, and so on down
+  // with its children in that order (see above), the child records of a
+  // record are a run, and so on down
   x.drec_off.assign(D + 1, 0);
   x.rbase = x.lneed;
   while (x.rbase < D && x.n_nonleaf[x.rbase] < kRestrictBase) x.rbase++;
   if (x.rbase == D) x.rbase = -1;
+  std::vector<int> drec;
   if (x.rbase >= 0) {
     const int nbase = x.n_nonleaf[x.rbase];
-    std::vector<int> drec(nbase + 1);
+    drec.resize(nbase + 1);
     for (int r = 0; r <= nbase; r++) drec[r] = r;
     for (int l = x.rbase; l + 1 < D; l++) {
       const std::vector<int>& down = nonleaf[l + 1];
-      for (int k = 0; k < x.n_nonleaf[l]; k++)
-        if (rchild[(size_t)x.rec_off[l] + k] != x.off[l + 1] + k * nch) ok = false;
       x.drec_off[l + 1] = (int)drec.size();
       for (int r = 0; r <= nbase; r++) {
         const int k = drec[(size_t)x.drec_off[l] + r];
         drec.push_back((int)(std::lower_bound(down.begin(), down.end(), k * nch) - down.begin()));
       }
     }
-    if (!ok) return bmg::fail(BMG_ERR_ARG, "tree: children out of cache order");
-    TRY(upload(&x.drec, drec));
+    if (!ordered) return bmg::fail(BMG_ERR_ARG, "tree: children out of cache order");
+  }
+  {
+    // one array: an allocation and copy of its own costs a rebuild 25 us
+    const size_t nh = halo.size(), ne = x.halo_end.size();
+    halo.insert(halo.end(), x.halo_end.begin(), x.halo_end.end());
+    halo.insert(halo.end(), drec.begin(), drec.end());
+    TRY(upload(&x.halo, halo));
+    x.halo_end_d = x.halo + nh;
+    x.drec = x.halo_end_d + ne;
   }
   clk.mark("compile: tables: halo cells");
   // fine-face averages: halo_face (all levels in one launch) and the face
