@@ -113,7 +113,7 @@ struct bmg_grid {
     Stat stat;
     double sum;
   }* host = nullptr;
-  int npartial = 1024;
+  int npartial = kSumParts;  // blocks of the first stage of a sum
   bool allocated_precision[2] = {false, false};
   // profiling
   bool prof = false;
@@ -2864,7 +2864,7 @@ struct Visc {
                          (const double*)vbuf(g, g->depth, VS_RES + c), lf.ncell);
     TRY(check_launch());
     if (out) *out = s;
-    return nans ? fail(BMG_ERR_NAN, "viscous residual is NaN") : BMG_OK;
+    return nans ? fail(BMG_ERR_NAN, "viscous residual is NaN (%llu values)", nans) : BMG_OK;
   }
 
   // mg_cycle (poisson.h:32-90) with minlevel 0 and relax_viscosity in the
@@ -2974,7 +2974,7 @@ struct Visc {
     }
     s.minlevel = 0;
     if (out) *out = s;
-    return nans ? fail(BMG_ERR_NAN, "viscous residual is NaN") : BMG_OK;
+    return nans ? fail(BMG_ERR_NAN, "viscous residual is NaN (%llu values)", nans) : BMG_OK;
   }
 };
 

@@ -1765,7 +1765,7 @@ int compile(bmg_tree* t) {
     if (nv) HIPCHECK(hipMemcpy(t->bcv[s], t->bc_host[s].data(), sizeof(double) * nv, hipMemcpyHostToDevice));
   }
   TRY(dalloc_((void**)&t->stat, sizeof(TStat)));
-  TRY(dalloc_((void**)&t->part, sizeof(double) * 1024));
+  TRY(dalloc_((void**)&t->part, sizeof(double) * kSumParts));
   TRY(dalloc_((void**)&t->scalar, sizeof(double)));
   t->compiled = true;
   // restore leaf values set before the mesh changed
@@ -2395,7 +2395,7 @@ int coefs(bmg_tree* t) {
 
 int sum_b(bmg_tree* t, double* out) {
   const DevIndex& x = t->ix;
-  int np = (int)std::min<long>(1024, std::max<long>(1, (long)nb_(x.nleaf)));
+  int np = (int)std::min<long>(kSumParts, std::max<long>(1, (long)nb_(x.nleaf)));
   k_t_sum_partial<<<np, kB, 0, t->stream>>>(x.leaf_gs, x.nleaf, t->b, t->part);
   k_t_sum_final<<<1, kB, 0, t->stream>>>(t->part, np, t->host ? &t->host->sum : t->scalar);
   if (!t->host) HIPCHECK(hipMemcpyAsync(out, t->scalar, sizeof(double), hipMemcpyDeviceToHost, t->stream));

@@ -490,7 +490,7 @@ __global__ __launch_bounds__(kViscThreads<DIM>) void k_visc_coarse(ViscCoarse A)
 }
 
 // residual_viscosity on the finest level: res = r - u + dt/rho S / D^2,
-// max |res| over the components to st (NaN counted)
+// max |res| over the components and the number of NaN to `part`
 // (per block partials, which k_reduce_stat folds, instead of 8192 atomic max
 // on one word: 106 -> 75 us at 128^3, 218 MB)
 template <int DIM>

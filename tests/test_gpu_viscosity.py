@@ -267,11 +267,26 @@ def test_viscosity_coarse_workgroup_bitexact(dim, depth):
         assert np.array_equal(ug[c], uo[c]), c
 
 
-def test_viscosity_counts_nan():
-    print("case viscosity nan", flush=True)
-    u, mu, rho = _problem(3, 4, 5, False)
-    u[1][3, 4, 5] = np.nan
-    g = bmg.Grid(3, 4)
-    g.set_niter(2)
-    with pytest.raises(bmg.BMGError):
-        g.viscosity(u, mu=mu, rho=rho, dt=0.01)
+@pytest.mark.parametrize("dim,depth,at", [(2, 2, (0, 3)), (2, 6, (17, 40)), (3, 4, (3, 4, 5)), (3, 5, (31, 0, 7))])
+@pytest.mark.parametrize("cycles", [0, 1])
+def test_viscosity_counts_nan(dim, depth, at, cycles):
+    """The NaN values of every residual of a solve are counted, over all
+    components and blocks: one NaN of the velocity against the residuals of
+    the oracle's cycle."""
+    print("case viscosity nan", dim, depth, cycles, flush=True)
+    u, mu, rho = _problem(dim, depth, 5, True)
+    u[1][at] = np.nan
+    o = Viscosity(dim, depth)
+    o.smoother = "rbgs"
+    o.set_coefficients(mu, rho)
+    res, _ = o.residual(u, u, 0.01)
+    count = sum(int(np.isnan(x).sum()) for x in res)
+    assert 0 < count < sum(x.size for x in res) or depth == 2
+    if cycles:
+        res, _ = o.residual(o.mg_cycle(u, res, 0.01, 4), u, 0.01)
+        count += sum(int(np.isnan(x).sum()) for x in res)
+    g = bmg.Grid(dim, depth)
+    g.set_niter(cycles, cycles)
+    with pytest.raises(bmg.BMGError, match=r"viscous residual is NaN \(%d values\)" % count) as e:
+        g.viscosity([x.copy() for x in u], mu=mu, rho=rho, dt=0.01)
+    assert e.value.code == 5
