@@ -673,11 +673,10 @@ int emb_check(const bmg_grid* g, int minlevel) {
 
 // --- kernels per dimension / precision --------------------------------
 
-// relax kernel of a level: the two-launch in-place red-black, the
-// single-pass streaming red-black (3D, n >= 128) or Jacobi
-// relax kernel of a level: two-launch in-place red-black (tiny levels),
-// one-launch fused red-black, single-pass streaming red-black (3D,
-// n >= 128) or Jacobi
+// relax kernel of a level: two-launch in-place red-black (tiny levels and
+// periodic 3D ones of n >= 128), red-black by tiles (2D, 3D up to n = 64),
+// single-pass streaming red-black (3D, n >= 128), one-launch fused red-black
+// (BMG_FUSED_MIN), Jacobi, Gauss-Seidel, embedded boundaries
 enum { RK_INPLACE_RB, RK_FUSED_RB, RK_STREAM_RB, RK_STREAM2_RB, RK_STREAM3_RB, RK_PAIR_RB, RK_TILE_RB, RK_JACOBI, RK_GS,
        RK_EMBED };
 
@@ -743,29 +742,22 @@ int level_kernel(const bmg_grid* g, int l) {
   const size_t nc = g->L[l].ncell;
   if (nc >= size_knob("BMG_FUSED_MIN", ~(size_t)0) && nc < size_knob("BMG_INPLACE_MIN", 1u << 20))
     return RK_FUSED_RB;
-  const bool tile = DIM == 2 || (DIM == 3 && (size_t)g->L[l].n <= size_knob("BMG_TILE_MAX3", 64));
+  // 2D: every level from 16^2 on (whole solves from memory take 1.8 to 2.6
+  // times as long from 1024^2 to 8192^2, both precisions; 13 cycles at 4096^2
+  // with a face field, FP64: 22.4 against 9.1 ms).  3D: up to 64^3 (11 us for
+  // two sweeps, FP32; in place 16 and 6 us of prolongation); at 128^3
+  // recomputing the halos costs more than the launches (25 against 24 us a
+  // sweep).
+  const bool tile = DIM == 2 || (DIM == 3 && g->L[l].n <= 64);
   return tile && g->rb_override < 0 && g->L[l].n >= 16 ? RK_TILE_RB : RK_INPLACE_RB;
 }
 
-// k_rb_tile on an n^DIM level: the region (a variant of the kernel) and the
-// sweeps per launch.  2D: up to 4 sweeps per launch (two launches of 2 take
-// 39 instead of 28 us at 1024^2, FP64), on the smallest region that leaves
-// the level at most about two workgroups per CU.  3D: 2 sweeps on 16^3 cells
-// (one sweep per launch: 15 instead of 11 us for two on 32^3 and 64^3, FP32;
-// the in-place kernel 16 us and 6 us of prolongation); at 128^3 recomputing
-// the halos costs more than the launches (25 against 24 us a sweep).
+// k_rb_tile, sweeps per launch.  2D: up to 4 (two launches of 2 take 39
+// instead of 28 us at 1024^2, FP64).  3D: 2 (one per launch: 15 instead of 11
+// us for two on 32^3 and 64^3, FP32; whole solves of 64^3 with face fields
+// 1.69 instead of 1.51 ms in FP64, 1.40 instead of 1.21 mixed).
 template <int DIM>
-int tile_variant(int n) {
-  if (DIM == 2) return n <= 256 ? 0 : n <= 512 ? 1 : 2;
-  return n <= 64 ? 0 : 1;
-}
-
-template <int DIM>
-int tile_sweeps(int n) {
-  const int dflt = DIM == 2 ? 4 : n <= 64 ? 2 : 1;
-  const size_t v = size_knob("BMG_TILE_SWEEPS", dflt);
-  return v >= 1 && v <= (DIM == 2 ? 4u : 2u) ? (int)v : dflt;
-}
+constexpr int kTileSweeps = DIM == 2 ? 4 : 2;
 
 // planes per workgroup of the streaming kernels (BMG_STREAM_CHUNK overrides,
 // a power of two dividing n)
@@ -1116,10 +1108,11 @@ int tile_sweep(bmg_grid* g, int l, int ns, int src, int dst, bool correct) {
   };
   ProfScope ps(g, l == g->depth ? PROF_RELAX_TILE : PROF_RELAX_COARSE);
   const bool af = k.lo[0] != nullptr;
-  [[maybe_unused]] const int v = tile_variant<DIM>(lv.n);
   if constexpr (DIM == 2) {
-    if (v == 0) af ? go(k_rb_tile<2, T, true, 16, 16, 1>, 16, 16, 1) : go(k_rb_tile<2, T, false, 16, 16, 1>, 16, 16, 1);
-    else if (v == 1) af ? go(k_rb_tile<2, T, true, 24, 24, 1>, 24, 24, 1)
+    // 32^2, 48^2 or 64^2 cells: the smallest that leaves a level of up to
+    // 1024^2 at most about two workgroups per CU
+    if (lv.n <= 256) af ? go(k_rb_tile<2, T, true, 16, 16, 1>, 16, 16, 1) : go(k_rb_tile<2, T, false, 16, 16, 1>, 16, 16, 1);
+    else if (lv.n <= 512) af ? go(k_rb_tile<2, T, true, 24, 24, 1>, 24, 24, 1)
                         : go(k_rb_tile<2, T, false, 24, 24, 1>, 24, 24, 1);
     else af ? go(k_rb_tile<2, T, true, 32, 32, 1>, 32, 32, 1) : go(k_rb_tile<2, T, false, 32, 32, 1>, 32, 32, 1);
   } else if constexpr (DIM == 3) {
@@ -1172,7 +1165,7 @@ int mg_cycle_t(bmg_grid* g, int nrelax, int minlevel, int maxlevel, bool defer) 
       // launches ping-pong between the buffers and end in da[0]; the first
       // one interpolates the initial guess, the last one of a cycle that
       // corrects by itself adds the correction
-      const int nl = (nrelax + tile_sweeps<DIM>(lv.n) - 1) / tile_sweeps<DIM>(lv.n);
+      const int nl = (nrelax + kTileSweeps<DIM> - 1) / kTileSweeps<DIM>;
       const bool own = l == g->depth && !(defer && maxlevel == g->depth);
       if (l == minlevel)
         hipLaunchKernelGGL((k_fill<T>), dim3(nblocks(lv.ncell)), dim3(kBlock), 0, g->stream, (T*)lv.da[nl & 1],

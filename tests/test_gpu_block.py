@@ -55,6 +55,14 @@ def test_levels_bitexact(dim, depth, box, precision, monkeypatch):
     _same(dim, depth, box, "alpha lam", precision, 4, (0, 1), monkeypatch)
 
 
+# levels of several hundred tiles of 64^2 cells
+@pytest.mark.parametrize("depth,box,coef,precision", [(11, "walls", "alpha", "fp64"), (11, "periodic", "lam", "mixed"),
+                                                      (11, "channel", "alpha lam", "fp64"),
+                                                      (12, "channel", "alpha", "mixed")])
+def test_large_2d_levels_bitexact(depth, box, coef, precision, monkeypatch):
+    _same(2, depth, box, coef, precision, 4, (1,), monkeypatch)
+
+
 @pytest.mark.parametrize("coef", ["alpha", "lam", ""])
 @pytest.mark.parametrize("dim,depth", [(2, 7), (3, 5)])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
