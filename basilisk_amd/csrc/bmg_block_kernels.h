@@ -20,7 +20,7 @@
 // LDS reads: 1.4 us instead of 0.6 us for a half-sweep of 4096 cells).
 #pragma once
 
-#include "bmg_kernels.h"
+#include "bmg_cells.h"
 
 namespace bmg {
 

@@ -16,137 +16,9 @@
 // compiled with -ffp-contract=off so that the FP64 path reproduces the CPU
 // oracle bit for bit.
 #pragma once
-#include <hip/hip_runtime.h>
-#include <stdint.h>
+#include "bmg_cells.h"
 
 namespace bmg {
-
-constexpr int kBlock = 256;
-
-// homogeneous boundary description of one level
-struct BCH {
-  int periodic[3];
-  int sigma[6];  // right, left, top, bottom, front, back
-  int tree;      // edge/corner ghosts by the tree rule (see bilinear_at)
-};
-
-// inhomogeneous boundary of `a` on the finest level: ghost = c + sigma * s,
-// with the cell size (x / Delta is computed as x * invD when Delta is a
-// power of two, which rounds identically)
-struct BCA {
-  int periodic[3];
-  int sigma[6];
-  const double* c[6];  // n^(DIM-1) values per side, or null for 0
-  double invD;
-  int pow2;
-};
-
-// cell indices fit in 32 bits (at most 2^30 cells per level)
-using idx_t = uint32_t;
-
-// two adjacent values as one vector load/store
-template <typename T>
-struct Vec2;
-template <>
-struct Vec2<float> {
-  using type = float2;
-};
-template <>
-struct Vec2<double> {
-  using type = double2;
-};
-
-
-template <int DIM>
-struct Geo {
-  int n, log2n;
-  __device__ __forceinline__ void decode(idx_t idx, int c[3]) const {
-    const idx_t m = (idx_t)(n - 1);
-    if (DIM == 3) {
-      c[2] = (int)(idx & m);
-      c[1] = (int)((idx >> log2n) & m);
-      c[0] = (int)(idx >> (2 * log2n));
-    } else if (DIM == 2) {
-      c[2] = 0;
-      c[1] = (int)(idx & m);
-      c[0] = (int)(idx >> log2n);
-    } else {
-      c[0] = (int)idx;
-      c[1] = c[2] = 0;
-    }
-  }
-  __device__ __forceinline__ idx_t stride(int d) const {
-    if (DIM == 3) return d == 0 ? (idx_t)1 << (2 * log2n) : d == 1 ? (idx_t)1 << log2n : 1u;
-    if (DIM == 2) return d == 0 ? (idx_t)1 << log2n : 1u;
-    return 1u;
-  }
-  __device__ __forceinline__ idx_t index(const int c[3]) const {
-    if (DIM == 3) return ((((idx_t)c[0] << log2n) + (idx_t)c[1]) << log2n) + (idx_t)c[2];
-    if (DIM == 2) return ((idx_t)c[0] << log2n) + (idx_t)c[1];
-    return (idx_t)c[0];
-  }
-  // index on the wall normal to d (tangential coordinates in order)
-  __device__ __forceinline__ idx_t wall(int d, const int c[3]) const {
-    if (DIM == 3)
-      return d == 0 ? ((idx_t)c[1] << log2n) + c[2] : d == 1 ? ((idx_t)c[0] << log2n) + c[2]
-                                                           : ((idx_t)c[0] << log2n) + c[1];
-    if (DIM == 2) return d == 0 ? (idx_t)c[1] : (idx_t)c[0];
-    return 0u;
-  }
-  __device__ __forceinline__ idx_t ncell() const { return (idx_t)1 << (DIM * log2n); }
-};
-
-// Blocks are dispatched round-robin over the 8 XCDs; give each XCD a
-// contiguous run of logical blocks so that neighbouring rows and planes of
-// a stencil share one L2.
-__device__ __forceinline__ idx_t logical_block() {
-  idx_t b = blockIdx.x, nb = gridDim.x;
-  if ((nb & 7) == 0) b = (b & 7) * (nb >> 3) + (b >> 3);
-  return b;
-}
-
-// index of the neighbour of cell c along d (dir +1 or -1): the cell itself
-// when the neighbour is a non-periodic ghost.  `ghost` tells which.
-template <int DIM>
-__device__ __forceinline__ idx_t nbr_index(const Geo<DIM>& g, const int* periodic, idx_t idx, const int c[3],
-                                           int d, int dir, bool& ghost) {
-  const idx_t s = g.stride(d);
-  const bool inside = dir > 0 ? c[d] < g.n - 1 : c[d] > 0;
-  const idx_t wrapoff = (idx_t)(g.n - 1) * s;
-  const idx_t step = dir > 0 ? idx + s : idx - s;
-  const idx_t wrapped = dir > 0 ? idx - wrapoff : idx + wrapoff;
-  ghost = !inside && !periodic[d];
-  return inside ? step : (periodic[d] ? wrapped : idx);
-}
-
-// value of field f at the neighbour of cell c along d (dir +1 or -1), with
-// the homogeneous ghost mapping (branch-free: a ghost reads the cell itself
-// and scales it by sigma)
-template <int DIM, typename T>
-__device__ __forceinline__ T nbr_h(const T* __restrict__ f, const Geo<DIM>& g, const BCH& bc, idx_t idx,
-                                   const int c[3], int d, int dir, T self) {
-  bool ghost;
-  idx_t iq = nbr_index<DIM>(g, bc.periodic, idx, c, d, dir, ghost);
-  T v = ghost ? self : f[iq];
-  return ghost ? T(bc.sigma[2 * d + (dir < 0)]) * v : v;
-}
-
-// alpha on the high face of cell c along d (one load from a selected address)
-template <int DIM, typename T>
-__device__ __forceinline__ T alpha_hi(const T* __restrict__ lo, const T* __restrict__ wall, const Geo<DIM>& g,
-                                      idx_t idx, const int c[3], int d) {
-  const T* p = c[d] < g.n - 1 ? lo + idx + g.stride(d) : wall + g.wall(d, c);
-  return *p;
-}
-
-template <typename T>
-struct Coef {
-  const T* lo[3];
-  const T* wall[3];
-  T alpha;        // used when lo[0] is null (constant alpha, unityf)
-  const T* lam;   // null: constant lam_c
-  T lam_c;
-};
 
 // n/d of the relax step, poisson.h:303-319
 template <int DIM, typename T>
@@ -514,23 +386,6 @@ __device__ __forceinline__ void axis_pair(const G& gc, const BCH& bc, int d, int
   off1 = (idx_t)qm * s;
 }
 
-// a ghost cell outside along two or three dimensions, from the value v of
-// the interior cell diagonal to it.  Multigrid (grid/multigrid.h:543-594,
-// one reflection per direction): the product of the sigmas times v.  Tree
-// (grid/tree.h:1168-1258): b1 + b2 - v, or b1 + b2 + b3 - 2 v, with
-// b = sigma v per crossed side (sums of +-v, so exact in any order).
-template <typename T>
-__device__ __forceinline__ T corner2(T v, T sa, T sb, bool tree) {
-  return tree ? (sb * v + sa * v) - v : (sa * sb) * v;
-}
-template <typename T>
-__device__ __forceinline__ T corner3(T v, T sx, T sy, T sz, bool gx, bool gy, bool gz, bool tree) {
-  int k = (int)gx + (int)gy + (int)gz;
-  if (!tree || k < 2) return ((sx * sy) * sz) * v;
-  if (k == 2) return ((gz ? sz * v : T(0)) + (gy ? sy * v : T(0)) + (gx ? sx * v : T(0))) - v;
-  return ((sz * v + sy * v) + sx * v) - T(2) * v;
-}
-
 // bilinear value at fine cell c from the coarse level,
 // grid/multigrid-common.h:124-140, child offsets grid/multigrid.h:175-188
 template <int DIM, typename T, typename G>
@@ -682,7 +537,7 @@ __global__ __launch_bounds__(kBlock) void k_coef_grad(const double* __restrict__
   out[t] = v;
 }
 
-[[maybe_unused]] static __global__ __launch_bounds__(kBlock) void k_lambda_grad(const double* __restrict__ a, const double* __restrict__ psi,
+__global__ __launch_bounds__(kBlock) void k_lambda_grad(const double* __restrict__ a, const double* __restrict__ psi,
                                                         double* __restrict__ out, size_t n) {
   size_t t = (size_t)blockIdx.x * kBlock + threadIdx.x;
   if (t < n) out[t] = -psi[t] * a[t];
@@ -696,7 +551,7 @@ struct Stat {
   unsigned long long nans;     // number of NaN residuals
 };
 
-[[maybe_unused]] static __global__ void k_stat_reset(Stat* s) {
+__global__ void k_stat_reset(Stat* s) {
   if (threadIdx.x == 0) {
     s->maxbits = 0ull;
     s->nans = 0ull;
@@ -811,7 +666,7 @@ __global__ __launch_bounds__(kBlock) void k_residual(const double* __restrict__ 
 }
 
 // deterministic two-stage sum (sum of b, poisson.h:163-167)
-[[maybe_unused]] static __global__ __launch_bounds__(kBlock) void k_sum_partial(const double* __restrict__ x, size_t n,
+__global__ __launch_bounds__(kBlock) void k_sum_partial(const double* __restrict__ x, size_t n,
                                                         double* __restrict__ part) {
   __shared__ double sh[kBlock / 64];
   double v = 0.;
@@ -829,7 +684,7 @@ __global__ __launch_bounds__(kBlock) void k_residual(const double* __restrict__ 
 // (the partials, at most kSumParts, come from LDS: one thread reading them
 // from memory one by one took 66 us for 1024)
 constexpr int kSumParts = 1024;
-[[maybe_unused]] static __global__ __launch_bounds__(kBlock) void k_sum_final(const double* __restrict__ part, int np,
+__global__ __launch_bounds__(kBlock) void k_sum_final(const double* __restrict__ part, int np,
                                                       double* __restrict__ out) {
   __shared__ double sh[kSumParts];
   for (int i = threadIdx.x; i < np; i += kBlock) sh[i] = part[i];
@@ -1009,7 +864,7 @@ __global__ __launch_bounds__(kBlock) void k_centered_gradient(CenteredArgs A, Ge
 }
 
 // correction (centered.h:322-327): u.x[] += dt*g.x[]
-[[maybe_unused]] static __global__ __launch_bounds__(kBlock) void k_correction(double* __restrict__ u, const double* __restrict__ gx,
+__global__ __launch_bounds__(kBlock) void k_correction(double* __restrict__ u, const double* __restrict__ gx,
                                                        double dt, size_t n) {
   const size_t idx = (size_t)blockIdx.x * kBlock + threadIdx.x;
   if (idx < n) u[idx] += dt * gx[idx];
@@ -1151,7 +1006,7 @@ struct ConvBatch {
   int nseg;
 };
 
-[[maybe_unused]] static __global__ __launch_bounds__(kBlock) void k_convert_batch(ConvBatch B) {
+__global__ __launch_bounds__(kBlock) void k_convert_batch(ConvBatch B) {
   const unsigned blk = blockIdx.x;
   // the segment of this block: the number of later segments starting at or
   // before it (independent loads of the increasing starts, not a chain)
@@ -1287,7 +1142,7 @@ __global__ __launch_bounds__(kBlock) void k_residual_restrict(const double* __re
   }
 }
 
-[[maybe_unused]] static __global__ __launch_bounds__(1024) void k_reduce_stat(const Part* __restrict__ part, int np, Stat* st) {
+__global__ __launch_bounds__(1024) void k_reduce_stat(const Part* __restrict__ part, int np, Stat* st) {
   __shared__ double smax[16];
   __shared__ unsigned long long snan[16];
   double m = 0.;
@@ -2523,27 +2378,6 @@ void k_corr_residual3(const double* __restrict__ a, const TD* __restrict__ da, d
 // then from minlevel up to top the zero / bilinear initial guess and nrelax
 // sweeps, with a block barrier between steps.  Same arithmetic as the
 // per-level kernels.
-
-// levels 0..12 at most (4096 cells in 1D)
-constexpr int kCoarseLevels = 13;
-
-template <typename T, int DIM>
-struct CoarseLevel {
-  T* da;
-  T* da2;  // Jacobi output
-  T* res;
-  Coef<T> k;
-  Geo<DIM> g;
-  BCH bc;
-  T D2;
-};
-
-template <typename T, int DIM>
-struct CoarseArgs {
-  CoarseLevel<T, DIM> L[kCoarseLevels];
-  int minlevel, top, nrelax, jacobi, gs;  // gs: the in-place Gauss-Seidel order, through da2
-  double* a;  // k_coarse_rb: where the finest level ends the cycle, the solution it corrects (or null)
-};
 
 template <int DIM, typename T>
 __device__ void coarse_relax_cell(const CoarseLevel<T, DIM>& L, idx_t idx, int colour_or_jacobi) {

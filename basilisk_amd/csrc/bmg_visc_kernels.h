@@ -31,6 +31,7 @@
 #include <hip/hip_runtime.h>
 
 #include "bmg_block_kernels.h"
+#include "bmg_kernels.h"
 
 namespace bmg {
 
