@@ -1234,24 +1234,25 @@ int compile(bmg_tree* t) {
     const long h = halo_of(l, v);
     if (h >= 0) __atomic_store_n(&stage[(size_t)h], (uint8_t)1, __ATOMIC_RELAXED);
   };
-  auto reads = [&](int l, int slot) {
-    if (slot >= hbase[l]) mark(l, entry(l, slot));
-    return slot;
-  };
   // active neighbours and colours
   long NA = x.abase[D] + x.nA[D];
   table<int> nbr((size_t)NA * 2 * dim);
   table<uint8_t> colour(NA);
   for (int l = 0; l <= D; l++)
     par_for((size_t)x.nA[l], [&](size_t q0, size_t q1) {
+      const int first = hbase[l];
+      auto reads = [&](int v) {
+        if (v >= first) mark(l, entry(l, v));
+        return v;
+      };
       for (size_t q = q0; q < q1; q++) {
         IJK c = T.active[l][q];
         size_t ai = (size_t)x.abase[l] + q;
         for (int d = 0; d < dim; d++) {
           int o[3] = {0, 0, 0};
           o[d] = 1;
-          nbr[ai * 2 * dim + 2 * d] = reads(l, chk(S(l, c.i - o[0], c.j - o[1], c.k - o[2])));
-          nbr[ai * 2 * dim + 2 * d + 1] = reads(l, chk(S(l, c.i + o[0], c.j + o[1], c.k + o[2])));
+          nbr[ai * 2 * dim + 2 * d] = reads(chk(S(l, c.i - o[0], c.j - o[1], c.k - o[2])));
+          nbr[ai * 2 * dim + 2 * d + 1] = reads(chk(S(l, c.i + o[0], c.j + o[1], c.k + o[2])));
         }
         colour[ai] = (uint8_t)((c.i + c.j + c.k) & 1);
       }
@@ -1276,16 +1277,17 @@ int compile(bmg_tree* t) {
           if (S(l + 1, 2 * c.i - GH + a, 2 * c.j - GH + b, dim == 3 ? 2 * c.k - GH + e : 0) != c0 + m)
             ok.store(false, std::memory_order_relaxed);
     int e0 = dim == 3 ? -1 : 0, e1 = dim == 3 ? 1 : 0;
-    size_t w = r * NR;
+    const int first = hbase[l];
+    int* ring = rring.data() + r * NR;
     for (int a = -1; a <= 1; a++)
       for (int b = -1; b <= 1; b++)
         for (int e = e0; e <= e1; e++) {
           int v = chk(S(l, c.i + a, c.j + b, c.k + e));
-          if (v >= hbase[l]) {
+          if (v >= first) {
             v = entry(l, v);
             if (read) mark(l, v);
           }
-          rring[w++] = v;
+          *ring++ = v;
         }
   };
   for (int l = 0; l <= D; l++) {
@@ -1356,7 +1358,12 @@ int compile(bmg_tree* t) {
         if (f.flags & (1 << d)) {
           int m[3] = {fc[0], fc[1], fc[2]};
           m[d]--;
-          FaceOp op = {reads(l, chk(S(l, fc[0], fc[1], fc[2]))), reads(l, chk(S(l, m[0], m[1], m[2]))), d};
+          FaceOp op = {chk(S(l, fc[0], fc[1], fc[2])), chk(S(l, m[0], m[1], m[2])), d};
+          // (next to an active cell both sides are marked by its neighbours)
+          if (std::min(op.gs, op.gm) >= hbase[l]) {
+            mark(l, entry(l, op.gs));
+            mark(l, entry(l, op.gm));
+          }
           fops[lp++] = op;
           fv_gs[g] = op.gs;
           fv_d[g++] = d;
@@ -1394,10 +1401,13 @@ int compile(bmg_tree* t) {
         }
         pos[m][k] = p;
       }
-    auto terms = [&](int l, size_t h, auto&& f) {  // the ring entries halo cell h of level l is interpolated from
+    // the ring entries, other than active cells, that halo cell h of level l
+    // is interpolated from
+    auto terms = [&](int l, size_t h, auto&& f) {
       const size_t r = (size_t)x.rec_off[l - 1] + x.n_nonleaf[l - 1] + (h >> dim);
-      const int* at = pos[h & (size_t)(nch - 1)];
-      for (int k = 0; k < nch; k++) f(rring[r * NR + at[k]]);
+      const int *ring = rring.data() + r * NR, *at = pos[h & (size_t)(nch - 1)], first = hbase[l - 1];
+      for (int k = 0; k < nch; k++)
+        if (const int v = ring[at[k]]; v < 0 || v >= first) f(v);
     };
     for (int l = D; l >= 1; l--)
       par_for(hoff[l + 1] - hoff[l], [&](size_t h0, size_t h1) {
