@@ -127,20 +127,23 @@ def _coarse_launches(dim, depth, top, nrelax):
     return n
 
 
-@pytest.mark.parametrize("dim,depth,coef,precision,default,top",
-                         [(2, 7, "alpha", "fp64", 5, t) for t in (0, 2, 6)] + [(2, 7, "lam", "mixed", 5, 4)]
-                         + [(3, 5, "alpha", "fp64", 3, t) for t in (1, 4)]
-                         + [(3, 5, "", "fp64", 4, 3), (3, 5, "alpha", "mixed", 4, 2)])
-def test_coarse_top_switch(dim, depth, coef, precision, default, top, monkeypatch):
+@pytest.mark.parametrize("dim,depth,box,coef,precision,default,top",
+                         [(2, 7, "walls", "alpha", "fp64", 5, t) for t in (0, 2, 6)]
+                         + [(2, 7, "channel", "lam", "mixed", 5, 4), (2, 7, "periodic", "alpha", "fp64", 5, 2)]
+                         + [(3, 5, "walls", "alpha", "fp64", 3, t) for t in (1, 4)]
+                         + [(3, 5, "walls", "", "fp64", 4, 3), (3, 5, "channel", "alpha", "mixed", 4, 2),
+                            (3, 5, "periodic", "", "mixed", 4, 2)])
+def test_coarse_top_switch(dim, depth, box, coef, precision, default, top, monkeypatch):
     """BMG_COARSE_TOP moves the level up to which a cycle runs in one
-    workgroup, also beyond what k_coarse_rb takes, with the same values."""
-    print("block coarse top", dim, depth, coef, precision, top, flush=True)
+    workgroup, also beyond what k_coarse_rb takes (tiles then run levels down
+    to 16 cells across, smaller than their region), with the same values."""
+    print("block coarse top", dim, depth, box, coef, precision, top, flush=True)
     out = []
     for t in (None, top):
         monkeypatch.delenv("BMG_COARSE_TOP", raising=False)
         if t is not None:
             monkeypatch.setenv("BMG_COARSE_TOP", str(t))
-        g = _grid(dim, depth, "walls", coef, precision)
+        g = _grid(dim, depth, box, coef, precision)
         g.residual()
         g.mg_cycle(4, 0)
         g.profile(True)
