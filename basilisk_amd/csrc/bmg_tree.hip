@@ -2092,7 +2092,7 @@ struct Batcher {
     C.minlevel = minlevel;
     C.top = top;
     C.nrelax = nrelax;
-    for (int l = minlevel; l <= top; l++) {
+    for (int l = 0; l <= top; l++) {
       C.off[l] = x.off[l];
       C.abase[l] = x.abase[l];
       const T D = (T)delta(t, l);
@@ -2332,10 +2332,10 @@ int cycle_kernels(bmg_tree* t, int nrelax, int minlevel, int maxlevel) {
   T* da = F<T>(t->da);
   Batcher<T, DIM> B(t, da, F<T>(t->res), F<T>(t->tmp));
   minlevel = std::min(minlevel, maxlevel);
-  // restriction (res) of mg_cycle: relax reads res in the cells it relaxes,
-  // so neither levels above minlevel nor halo cells nor ghosts
+  // restriction (res) of mg_cycle, to every level (relax() may read those
+  // below minlevel afterwards), but to neither halo cells nor ghosts
   const int top = B.coarse_top(minlevel, maxlevel);
-  const int rlow = std::max(minlevel, top);
+  const int rlow = std::max(0, top);
   if (x.depth > rlow) B.restrict_range(1, x.depth - 1, rlow);
   if (top >= 0) B.coarse(nrelax, minlevel, top);
   for (int l = top >= 0 ? top + 1 : minlevel; l <= maxlevel; l++) {

@@ -50,7 +50,8 @@ __global__ __launch_bounds__((bmg::kCoarseThreads<DIM, T, ALPHAF>)) void k_t_coa
   __shared__ T big[NC * kBlocks], small[kBlocks], rs[2 * kBlocks];
   const int t = threadIdx.x;
   auto roff = [](int l) { return ((1 << (DIM * l)) - 1) / (NC - 1); };
-  for (int l = A.top - 1; l >= A.minlevel; l--) {
+  // (the levels below minlevel too: relax() may read their res)
+  for (int l = A.top - 1; l >= 0; l--) {
     for (int q = t; q < 1 << (DIM * l); q += (int)blockDim.x) {
       const T* c = l + 1 == A.top ? A.res + A.off[l + 1] + q * NC : rs + roff(l + 1) + q * NC;
       T sum = T(0);

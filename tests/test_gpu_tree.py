@@ -315,3 +315,26 @@ def test_relax_reads_ghosts_of_every_side(dim, depth):
     g.relax(depth)
     da = _numpy_relax(da, res, -1.25, ghosts, D, parity >= 0, True)
     assert np.array_equal(g.get_da(), da[at])
+
+
+@pytest.mark.parametrize("smoother", ["jacobi", "rbgs"])
+@pytest.mark.parametrize("dim,depth,minlevel", [(2, 6, 1), (2, 7, 2), (3, 4, 1), (3, 5, 2)])
+def test_cycle_restricts_the_residual_to_every_level(dim, depth, minlevel, smoother):
+    """mg_cycle restricts res to all levels (poisson.h:42), also those below
+    its minlevel, where relax() reads it: after cycles without relaxations,
+    from the root and from the finest level, relax() on each level agrees."""
+    print("cycle restricts", dim, depth, minlevel, smoother, flush=True)
+    got = []
+    for m in (0, 1, depth):
+        g = bmg.Tree(dim, 1.0, (0.0, 0.0, 0.0), smoother=smoother)
+        tree_cases.spheres_problem(g, depth, 11, nspheres=2, minlevel=minlevel)
+        g.restriction_alpha_lambda()
+        g.residual()
+        g.mg_cycle(0, m, depth)
+        out = []
+        for l in range(depth + 1):
+            g.relax(l)
+            out.append(g.get_da())
+        got.append(np.array(out))
+    assert np.abs(got[0]).max() > 0
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
