@@ -789,7 +789,9 @@ struct bmg_tree {
   double* bcv[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
   bool coef_ready = false;
   // the level whose boundary pass of da the last cycle left out (-1: none);
-  // only bmg_tree_relax reads what it would have written
+  // only bmg_tree_relax reads what it would have written.  It is made up for
+  // before a relax, before a cycle that ends on a coarser level and before
+  // the kind of a side changes.
   int da_level = -1;
   TStat* stat = nullptr;
   // pinned host memory that the reductions' last kernels write (null: copied
@@ -1943,8 +1945,8 @@ RelaxCoef<T> relax_coef(bmg_tree* t) {
 template <typename T, int DIM>
 void pending_boundary(bmg_tree* t);
 
-// one relax of level l (bmg_tree_relax): Jacobi reads the ghosts' stored
-// values, red-black evaluates their rules
+// one relax of level l (bmg_tree_relax): it reads the ghosts' stored values,
+// as the last boundary pass left them
 template <typename T, int DIM>
 int relax(bmg_tree* t, int l) {
   const DevIndex& x = t->ix;
@@ -1958,20 +1960,19 @@ int relax(bmg_tree* t, int l) {
   if (t->smoother == BMG_RELAX_JACOBI) {
     {
       TProf tp(t, seg_cells(S));
-      k_t_relax<T, DIM><<<nbk, kB, 0, t->stream>>>(S, da, F<T>(t->tmp), res, x.nbr, x.box, bct(t), k);
+      k_t_relax<T, DIM><<<nbk, kB, 0, t->stream>>>(S, da, F<T>(t->tmp), res, x.nbr, x.box, bct(t), k, 1);
     }
     k_t_jacobi<T><<<nbk, kB, 0, t->stream>>>(S, da, F<T>(t->tmp));
   } else if (t->smoother == BMG_RELAX_RBGS) {
     for (int c = 0; c < 2; c++) {
-      // the stored ghosts, which a Jacobi relax may read next (their sources
-      // are cells of the box: every level in one launch)
+      // (the ghosts' sources are cells of the box: every level in one launch)
       const int ng = x.box_off[l] + x.box_n[l];
       if (c && ng) k_t_box<T><<<nb_(ng), kB, 0, t->stream>>>(x.box, ng, da, bct(t), BK_HOM, t->L0);
       Segs SC = level_or_leaf_colour(t, l, c);
       unsigned nbc = (unsigned)SC.first_block[SC.n];
       if (nbc) {
         TProf tp(t, seg_cells(SC));
-        k_t_relax<T, DIM><<<nbc, kB, 0, t->stream>>>(SC, da, nullptr, res, x.nbr, x.box, bct(t), k);
+        k_t_relax<T, DIM><<<nbc, kB, 0, t->stream>>>(SC, da, nullptr, res, x.nbr, x.box, bct(t), k, 1);
       }
     }
   } else
@@ -2181,7 +2182,7 @@ struct Batcher {
       if (!nbc) continue;
       TProf tp(t, seg_cells(SC));
       k_t_relax<T, DIM><<<nbc, kB, 0, t->stream>>>(SC, da, jac ? A.fld[2] : nullptr, A.res, x.nbr, x.box, A.bc,
-                                                   A.k);
+                                                   A.k, 0);
     }
     if (jac) {
       Segs S = level_or_leaf(t, l);
@@ -2367,9 +2368,18 @@ void pending_boundary(bmg_tree* t) {
   t->da_level = -1;
 }
 
+// the same from the settings (a mesh that changed since has no da to keep)
+void pending_boundary(bmg_tree* t) {
+  if (t->da_level < 0 || !t->compiled || t->topo.dirty) return;
+  const bool mixed = t->precision == BMG_MIXED;
+  if (t->dim == 3) mixed ? pending_boundary<float, 3>(t) : pending_boundary<double, 3>(t);
+  else mixed ? pending_boundary<float, 2>(t) : pending_boundary<double, 2>(t);
+}
+
 template <typename T, int DIM>
 int mg_cycle(bmg_tree* t, int nrelax, int minlevel, int maxlevel) {
   TRY(coefficients<T, DIM>(t));
+  if (t->da_level > maxlevel) pending_boundary<T, DIM>(t);
   t->da_level = maxlevel;
   if (!t->use_graphs || t->prof) {
     TRY((cycle_kernels<T, DIM>(t, nrelax, minlevel, maxlevel)));
@@ -3212,6 +3222,7 @@ int bmg_tree_set_bc(bmg_tree* t, int side, int kind, const double* values) {
     for (int e = 1; e < t->dim; e++) p *= (1L << l);
     m += p;
   }
+  if (t->bc_kind[side] != kind) pending_boundary(t);
   t->bc_kind[side] = kind;
   drop_graphs(t);
   t->bc_host[side].assign(m, 0.);

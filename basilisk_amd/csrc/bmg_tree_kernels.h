@@ -295,10 +295,11 @@ struct RelaxCoef {
 // values do not wait for them: evaluated one after the other, each behind a
 // branch, they took 101 us of a Jacobi cycle of a 4^3 tree, now 59, and in
 // k_t_relax 7.2 us a launch on an FP64 octree of 36k leaves, now 4.7.
+// (stored: the ghosts' stored values instead, for a relax outside a cycle)
 template <typename T, int DIM>
 __device__ __forceinline__ T t_relax_value(const T* da, const BoxRule* __restrict__ box, const BCT& bc,
                                            const T* __restrict__ res, const int* __restrict__ nb,
-                                           const RelaxCoef<T>& k, int gs, T D2) {
+                                           const RelaxCoef<T>& k, int gs, T D2, bool stored = false) {
   int s[2 * DIM], any = 0;
   T v[2 * DIM];
 #pragma unroll
@@ -316,6 +317,7 @@ __device__ __forceinline__ T t_relax_value(const T* da, const BoxRule* __restric
       if (s[e] < 0) {
         s[e] = ghost;
         if ((dirichlet >> side) & 1) v[e] = -v[e];
+        if (stored) v[e] = da[ghost];
       }
     }
   }
@@ -337,7 +339,7 @@ __device__ __forceinline__ T t_relax_value(const T* da, const BoxRule* __restric
 template <typename T, int DIM>
 __global__ __launch_bounds__(kB) void k_t_relax(Segs S, T* da, T* __restrict__ out, const T* __restrict__ res,
                                                 const int* __restrict__ nbr, const BoxRule* __restrict__ box, BCT bc,
-                                                RelaxCoef<T> k) {
+                                                RelaxCoef<T> k, int stored) {
   int s = seg_of(S);
   int gs = seg_slot(S, s);
   if (gs < 0) return;
@@ -345,7 +347,7 @@ __global__ __launch_bounds__(kB) void k_t_relax(Segs S, T* da, T* __restrict__ o
   T D = (T)S.D[s];
   const int t = ((int)blockIdx.x - S.first_block[s]) * kB + (int)threadIdx.x;
   const int* nb = S.nbl[s] ? S.nbl[s] + (size_t)t * 2 * DIM : nbr + (size_t)ai * 2 * DIM;
-  T v = t_relax_value<T, DIM>(da, box, bc, res, nb, k, gs, D * D);
+  T v = t_relax_value<T, DIM>(da, box, bc, res, nb, k, gs, D * D, stored);
   if (out)
     out[gs] = v;
   else

@@ -281,19 +281,15 @@ def _numpy_relax(da, res, lam, ghosts, D, cells, jacobi):
     return np.where(cells, (da + 2.0 * w) / 3.0 if jacobi else w, da)
 
 
-@pytest.mark.parametrize("dim,depth", [(2, 1), (2, 3), (2, 6), (3, 1), (3, 2), (3, 4)])
-def test_relax_reads_ghosts_of_every_side(dim, depth):
-    """relax() on a full level with homogeneous Dirichlet, Neumann and
-    symmetric sides, bit for bit: red-black evaluates the ghosts, a Jacobi
-    relax after it reads the values stored between the colours."""
-    print("relax ghosts", dim, depth, flush=True)
+def _full_level(dim, depth):
+    """A full tree with every kind of side, its residual, and the grid index
+    of every leaf."""
     g = bmg.Tree(dim, 1.0, (0.0, 0.0, 0.0), smoother="rbgs")
     g.refine(lambda x, y, z, lev: lev < depth)
     n = 1 << depth
     _, xyz = g.leaves()
     at = tuple((xyz[:, c] * n).astype(int) for c in range(dim))
-    rng = np.random.default_rng(dim * 10 + depth)
-    b = rng.standard_normal((n,) * dim)
+    b = np.random.default_rng(dim * 10 + depth).standard_normal((n,) * dim)
     g.set_b(b[at].copy())
     g.set_a(np.zeros(len(xyz)))
     g.set_lambda(-1.25)
@@ -302,18 +298,60 @@ def test_relax_reads_ghosts_of_every_side(dim, depth):
     g.residual()
     res = np.empty_like(b)
     res[at] = g.get_res()
-    D, da = 1.0 / n, np.zeros_like(b)
+    return g, res, at
+
+
+@pytest.mark.parametrize("dim,depth", [(2, 1), (2, 3), (2, 6), (3, 1), (3, 2), (3, 4)])
+def test_relax_reads_ghosts_of_every_side(dim, depth):
+    """relax() on a full level with homogeneous Dirichlet, Neumann and
+    symmetric sides, bit for bit.  It reads the ghosts' stored values, which a
+    red-black relax stores between its colours and a Jacobi relax does not."""
+    print("relax ghosts", dim, depth, flush=True)
+    g, res, at = _full_level(dim, depth)
+    D, da = 1.0 / (1 << depth), np.zeros_like(res)
     g.mg_cycle(0, depth, depth)  # da = 0
-    parity = np.indices(b.shape).sum(0) & 1
-    for _ in range(3):
+    parity = np.indices(res.shape).sum(0) & 1
+    ghosts = da
+    for smoother in ("rbgs", "rbgs", "jacobi", "rbgs", "jacobi", "jacobi", "rbgs", "rbgs"):
+        g.set_smoother(smoother)
         g.relax(depth)
-        da = _numpy_relax(da, res, -1.25, da, D, parity == 0, False)
-        ghosts = da.copy()
-        da = _numpy_relax(da, res, -1.25, da, D, parity == 1, False)
-        assert np.array_equal(g.get_da(), da[at])
-    g.set_smoother("jacobi")
+        if smoother == "rbgs":
+            da = _numpy_relax(da, res, -1.25, ghosts, D, parity == 0, False)
+            ghosts = da.copy()
+            da = _numpy_relax(da, res, -1.25, ghosts, D, parity == 1, False)
+        else:
+            da = _numpy_relax(da, res, -1.25, ghosts, D, parity >= 0, True)
+        assert np.array_equal(g.get_da(), da[at]), smoother
+
+
+@pytest.mark.parametrize("between", ["other sides", "coarser cycle"])
+@pytest.mark.parametrize("dim,depth", [(2, 3), (2, 6), (3, 2), (3, 4)])
+def test_relax_reads_the_ghosts_of_the_last_cycle(dim, depth, between):
+    """The ghosts that relax() reads first are those of the cycle that last
+    reached its level: with the sides of that time, and also when a cycle of
+    the coarser levels followed."""
+    print("relax last cycle", dim, depth, between, flush=True)
+    g, res, at = _full_level(dim, depth)
+    D, da = 1.0 / (1 << depth), np.zeros_like(res)
+    parity = np.indices(res.shape).sum(0) & 1
+    g.mg_cycle(1, depth, depth)
+    for colour in (0, 1):
+        da = _numpy_relax(da, res, -1.25, da, D, parity == colour, False)
+    if between == "coarser cycle":
+        g.mg_cycle(2, 0, depth - 1)
+        g.set_smoother("jacobi")
+        da = _numpy_relax(da, res, -1.25, da, D, parity >= 0, True)
+    else:
+        old = list(SIDES)
+        red = _numpy_relax(da, res, -1.25, da, D, parity == 0, False)
+        try:
+            for side in range(2 * dim):
+                SIDES[side] = bmg.BC_NEUMANN if old[side] == bmg.BC_DIRICHLET else bmg.BC_DIRICHLET
+                g.set_bc(side, SIDES[side])
+            da = _numpy_relax(red, res, -1.25, red, D, parity == 1, False)
+        finally:
+            SIDES[:] = old
     g.relax(depth)
-    da = _numpy_relax(da, res, -1.25, ghosts, D, parity >= 0, True)
     assert np.array_equal(g.get_da(), da[at])
 
 
